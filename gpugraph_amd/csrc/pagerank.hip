@@ -8,12 +8,13 @@
 //           compensated FP32, fixed fold order), writing r_next and, unweighted, the contribution
 //           x = r_next / outdeg used by the next sweep; the same pass adds
 //           |r_next - r| and the dangling mass of r_next in FP64 (one atomic
-//           per workgroup).  A one-thread finalize kernel closes the
+//           per workgroup).  A one-wave finalize kernel closes the
 //           iteration on the device (residual, D, iteration count, done
 //           flag); sweeps early-exit once done, so the host checks the state
 //           only every kItersPerCheck iterations.
 // Adjoint:  for L = c^T r,  lambda = c + d (P lambda + delta (1^T lambda)/n)
 //           (the transposed fixed point: row reductions over CSR out-edges),
+//           its slow constant component removed at every sweep (PrAdjointOp),
 //           dL/dt = (1-d) lambda, and for raw weights
 //           dL/dw_uv = d r_u / S_u (lambda_v - sum_v' P_uv' lambda_v')
 //           (unweighted graphs: dL/dP_uv = d r_u lambda_v).  The forward
@@ -27,8 +28,8 @@
 // Byte model per sweep: unweighted 20n + 8m (+4n with a teleport vector):
 // per vertex offsets, old/new rank, new contribution, 1/outdeg; per edge
 // the source id and its contribution.  Weighted 16n + 12m (+4n): per edge
-// source id, P_uv and r_u.  Adjoint sweep 24n + 8m (weighted + 4m): per
-// vertex offsets, old/new lambda, c, row sum, 1/outdeg; per edge target id,
+// source id, P_uv and r_u.  Adjoint sweep 20n + 8m (weighted + 4m): per
+// vertex offsets, old/new lambda, c, 1/outdeg; per edge target id,
 // its lambda (and P_uv).  Gradient pass 16m + 16n.
 #include <hip/hip_runtime.h>
 
@@ -54,22 +55,39 @@ struct PrState {
   double aux_cur;             // dangling mass (forward) / sum of lambda (adjoint) of the current vector
   double scale;               // residual scale: 1 (forward) or ||c||_1 (adjoint)
   double resid_last;
+  double offset;              // adjoint: constant to add to the last vector (k_adj_finalize)
   int32_t iters, done;
+  int32_t plain_only, pad;    // adjoint: the shift has been given up for the rest of the run
+  double shift, gap;          // adjoint: sigma of the vector the next sweep reads, and that vector minus
+                              // the plain iterate (k_adj_finalize)
   // Per-workgroup FP64 sums, striped (see GASengine::block_counter_add):
   // accumulated by a sweep (or k_pr_init), folded by k_pr_finalize /
   // k_pr_start.
   double resid_acc[kStripes * kPrStride], aux_acc[kStripes * kPrStride], scale_acc[kStripes * kPrStride];
+  double sq_acc[kStripes * kPrStride];
 };
 
-// Fold a striped FP64 sum and clear its stripes (one thread).
+// Fold a striped FP64 sum and clear its stripes (one wave, a lane a stripe;
+// every lane gets the sum).  A single thread doing this is slower (16 loads
+// one by one) and not safe: its loads have a uniform address, so they may go
+// through the scalar cache, which is not ordered with the vector stores that
+// clear the same words.
 __device__ __forceinline__ double take_stripes(double *acc) {
+  static_assert(kStripes <= kWave, "a lane per stripe");
+  const int q = lane_id();
   double t = 0.0;
-  for (int q = 0; q < kStripes; q++) {
-    t += acc[q * kPrStride];
+  if (q < kStripes) {
+    t = acc[q * kPrStride];
     acc[q * kPrStride] = 0.0;
   }
-  return t;
+#pragma unroll
+  for (int off = kStripes / 2; off > 0; off >>= 1) t += __shfl_xor(t, off);
+  return __shfl(t, 0);
 }
+
+// Waits for the scalar loads issued so far: a state word read through the
+// scalar cache must have arrived before a vector store replaces it.
+__device__ __forceinline__ void scalar_loads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 template <int BLOCK>
 __device__ __forceinline__ void block_add_f64(double *p, double v) {
@@ -151,6 +169,22 @@ struct PrForwardOp {
   }
 };
 
+// Adjoint sweep, lambda' = c + d P (lambda + sigma 1) (P with its dangling
+// rows replaced by 1/n).  P 1 = 1, so a plain sweep shrinks the constant part
+// of the error by d only, while the rest goes down by d |lambda_2(P)|: on
+// R-MAT graphs 65-70 plain sweeps to a residual of 2e-7 ||c||_1, where the
+// forward iteration (whose error carries no mass) needs 14-19.  sigma removes
+// that part: the residual R = lambda' - lambda of a constant error s is
+// (1 - d) s, so k_adj_finalize adds sigma = d mean(R) / (1 - d) to the next
+// vector read.  The iteration then converges by the second eigenvalue (10-14
+// sweeps) for any start; sigma goes to 0 with the residual, so the fixed
+// point is unchanged.  sigma is added to the row sums (rows of P sum to 1),
+// one scalar per sweep: no vector is read or written for it.
+//
+// gap is lambda + sigma minus the plain iterate o of the same sweep number
+// (gap' = d gap + sigma), so this pass has both residuals: R_o = R + (1 - d)
+// gap, whose L1 norm is the plain iteration's stopping test, and the sum of
+// R^2 (k_adj_finalize says which ends the run).
 struct PrAdjointOp {
   const int32_t *off;   // CSR row offsets
   const int32_t *dst;   // CSR column indices
@@ -158,21 +192,25 @@ struct PrAdjointOp {
   const float *inv_out;
   float *lam[2];
   const float *c;
-  float *rowsum;        // sum_v P_uv lambda_v of the vector read by this sweep
   float d;
   double inv_n;
   PrState *st;
   const float *lc;  // this sweep's lambda and the next one (picked in begin())
   float *lnx;
-  float ln;
-  double resid, lsum;
+  float sigma, ln;
+  double shift, gamma;
+  double resid, sq, lsum;
 
   __device__ __forceinline__ void begin() {
     const bool odd = st->iters & 1;
     lc = odd ? lam[1] : lam[0];
     lnx = odd ? lam[0] : lam[1];
-    ln = (float)(st->aux_cur * inv_n);
+    shift = st->shift;
+    sigma = (float)shift;
+    gamma = (1.0 - (double)d) * st->gap;
+    ln = (float)(st->aux_cur * inv_n + shift);
     resid = 0.0;
+    sq = 0.0;
     lsum = 0.0;
   }
   __device__ __forceinline__ int32_t row_begin(int32_t u) { return off[u]; }
@@ -197,10 +235,11 @@ struct PrAdjointOp {
   __device__ __forceinline__ State vertex_state(int32_t u) { return {lc[u], inv_out[u], c[u]}; }
   __device__ __forceinline__ void item_done(int32_t u, float sum, const State &st) {
     const float su = pcsr ? sum : sum * st.io;
-    const float ln_u = st.cu + d * (su + (st.io == 0.0f ? ln : 0.0f));
+    const float ln_u = st.cu + d * (st.io == 0.0f ? ln : su + sigma);
     lnx[u] = ln_u;
-    rowsum[u] = su;
-    resid += fabs((double)ln_u - (double)st.l_old);
+    const double r = (double)ln_u - ((double)st.l_old + shift);
+    resid += fabs(r + gamma);
+    sq += r * r;
     lsum += ln_u;
   }
   // Per-edge form (XCD-sliced sweeps).
@@ -208,16 +247,85 @@ struct PrAdjointOp {
   __device__ __forceinline__ void item_done(int32_t u, float sum) { item_done(u, sum, vertex_state(u)); }
   __device__ __forceinline__ void finish() {
     block_add_f64<kRowBlock>(st->resid_acc, resid);
+    block_add_f64<kRowBlock>(st->sq_acc, sq);
     block_add_f64<kRowBlock>(st->aux_acc, lsum);
   }
 };
 
-__global__ void k_pr_finalize(PrState *st, double tol, int32_t max_iter) {
+// End of a forward sweep (one wave).
+__global__ void __launch_bounds__(kWave) k_pr_finalize(PrState *st, double tol, int32_t max_iter) {
   if (st->done) return;
-  st->resid_last = take_stripes(st->resid_acc);
-  st->aux_cur = take_stripes(st->aux_acc);
-  st->iters++;
-  if (st->resid_last <= tol * st->scale || st->iters >= max_iter) st->done = 1;
+  const double limit = tol * st->scale;
+  const int32_t iters = st->iters + 1;
+  const double resid = take_stripes(st->resid_acc), aux = take_stripes(st->aux_acc);
+  scalar_loads_done();
+  if (threadIdx.x != 0) return;
+  st->resid_last = resid;
+  st->aux_cur = aux;
+  st->iters = iters;
+  if (resid <= limit || iters >= max_iter) st->done = 1;
+}
+
+// End of an adjoint sweep.  Two tests end the run, whichever holds first:
+//  * sqrt(n sum R^2) <= tol ||c||_1 / 2: bounds the L1 residual, and bounds
+//    the error of parts that converge by d alone (small closed components) by
+//    half of what a residual spread evenly over the vertices leaves, which is
+//    the plain iteration's error: a bare L1 test would end on a few vertices
+//    with a large error, because the constant part no longer holds the run up
+//    (1.5e-5 relative against 7.6e-7 on an undirected R-MAT of scale 14).
+//    Relative errors of lambda against 64 bits, R-MAT of 0.7M vertices: 8e-7
+//    plain, at most 5e-7 so.  lambda' is the result.
+//  * the plain iteration's own test, L1 of R_o <= tol ||c||_1: a run never
+//    takes more sweeps than the plain iteration.  The result is then its
+//    iterate, lambda' - d gap (offset).
+// At max_iter the plain iterate and its residual are returned as well.
+// From sweep kShiftTrial on, a residual whose bound is not below the plain
+// iteration's own says that the rest converges no faster than the constant
+// part (|lambda_2| = 1: cycles, stars, several closed components); the run
+// then goes back to the plain iterate (sigma = -gap) and stays with it, since
+// a shifted vector keeps changing in its last bits where a plain one settles
+// (star of 1500 vertices: 90 sweeps with the shift to the end, 78 plain).
+// No shift once the residual's sum is at the rounding level of the FP32
+// vectors (2^-24 ||c||_1): both tests then see a settled iteration.
+constexpr int kShiftTrial = 16;
+__global__ void __launch_bounds__(kWave)
+k_adj_finalize(PrState *st, double tol, int32_t max_iter, int32_t n, double d) {
+  if (st->done) return;
+  const double limit = tol * st->scale, noise = 0x1p-24 * st->scale;
+  const double read = st->aux_cur + (double)n * st->shift;  // sum of the vector this sweep read
+  const double gap = d * st->gap;                           // lambda' minus the plain iterate
+  const int32_t iters = st->iters + 1;
+  bool plain_only = st->plain_only != 0;
+  const double plain = take_stripes(st->resid_acc), sq = take_stripes(st->sq_acc), sum = take_stripes(st->aux_acc);
+  scalar_loads_done();
+  if (threadIdx.x != 0) return;
+  const double bound = sqrt((double)n * sq), rsum = sum - read;
+  st->aux_cur = sum;
+  st->iters = iters;
+  const bool own = 2.0 * bound <= limit;
+  if (own || plain <= limit || iters >= max_iter) {
+    st->resid_last = own ? bound : plain;
+    st->offset = own ? 0.0 : -gap;
+    st->done = 1;
+    return;
+  }
+  if (iters >= kShiftTrial && bound >= plain) plain_only = true;
+  double shift = 0.0;
+  if (plain_only)
+    shift = -gap;
+  else if (isfinite(rsum) && fabs(rsum) > noise)
+    shift = d / (1.0 - d) * rsum / (double)n;
+  shift = (double)(float)shift;
+  st->resid_last = plain;
+  st->plain_only = plain_only;
+  st->shift = shift;
+  st->gap = gap + shift;
+}
+
+__global__ void k_add_offset(float *__restrict__ x, const PrState *__restrict__ st, int32_t n) {
+  const double a = st->offset;
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x)
+    x[v] = (float)((double)x[v] + a);
 }
 
 // Start vector (forward: teleport or uniform; adjoint: c) and its aux sum.
@@ -242,11 +350,13 @@ k_pr_init(float *r0, float *x0, const float *tele, const float *inv_out, int32_t
   block_add_f64<kRowBlock>(st->scale_acc, mag);
 }
 
-__global__ void k_pr_start(PrState *st, int adjoint) {
-  st->scale = take_stripes(st->scale_acc);
-  if (!adjoint || st->scale == 0.0) st->scale = 1.0;
-  st->aux_cur = take_stripes(st->aux_acc);
-  (void)take_stripes(st->resid_acc);
+__global__ void __launch_bounds__(kWave) k_pr_start(PrState *st, int adjoint) {
+  const double scale = take_stripes(st->scale_acc), aux = take_stripes(st->aux_acc);
+  if (threadIdx.x != 0) return;
+  st->scale = !adjoint || scale == 0.0 ? 1.0 : scale;
+  st->aux_cur = aux;
+  st->offset = st->shift = st->gap = 0.0;
+  st->plain_only = 0;
   st->resid_last = INFINITY;
   st->iters = 0;
   st->done = 0;
@@ -530,7 +640,7 @@ int stage_input(gg_graph *g, const float *p, uint32_t flags, gg::DevBuf &buf, co
 template <class Op>
 int iterate(gg_graph *g, Op op, int dir, const SliceLists *slices, PrState *st, double tol, int32_t max_iter,
             const char *kname, double bytes_per_sweep, int32_t *iters_out, double *resid_out,
-            double *scale_out = nullptr) {
+            double *scale_out = nullptr, double *offset_out = nullptr) {
   hipStream_t s = g->stream;
   const int32_t *done = &st->done;
   float2 *part = slices ? g->sl_part.as<float2>() : nullptr;
@@ -542,12 +652,13 @@ int iterate(gg_graph *g, Op op, int dir, const SliceLists *slices, PrState *st, 
     GG_TRY(g->seg_carry.ensure(sizeof(SegCarry) * (size_t)seg_tiles(g->n, g->m)));
     carry = g->seg_carry.as<SegCarry>();
   }
-  // Read back from PrState::scale on: scale, resid_last, iters, done.
+  // Read back from PrState::scale on: scale, resid_last, offset, iters, done.
   struct H {
-    double scale, resid_last;
+    double scale, resid_last, offset;
     int32_t iters, done;
   };
   static_assert(offsetof(PrState, resid_last) == offsetof(PrState, scale) + offsetof(H, resid_last) &&
+                    offsetof(PrState, offset) == offsetof(PrState, scale) + offsetof(H, offset) &&
                     offsetof(PrState, iters) == offsetof(PrState, scale) + offsetof(H, iters) &&
                     offsetof(PrState, done) == offsetof(PrState, scale) + offsetof(H, done),
                 "PrState read-back layout");
@@ -560,7 +671,10 @@ int iterate(gg_graph *g, Op op, int dir, const SliceLists *slices, PrState *st, 
         else
           seg_rows_launch(op, offs, g->n, g->m, parts, carry, done, g->opt.expand_grid, s);
       }
-      hipLaunchKernelGGL(k_pr_finalize, dim3(1), dim3(1), 0, s, st, tol, max_iter);
+      if (offset_out)
+        hipLaunchKernelGGL(k_adj_finalize, dim3(1), dim3(kWave), 0, s, st, tol, max_iter, g->n, (double)op.d);
+      else
+        hipLaunchKernelGGL(k_pr_finalize, dim3(1), dim3(kWave), 0, s, st, tol, max_iter);
     }
     GG_HIP(hipGetLastError());
     GG_HIP(hipMemcpyAsync(g->h_pinned, &st->scale, sizeof(H), hipMemcpyDeviceToHost, s));
@@ -571,6 +685,7 @@ int iterate(gg_graph *g, Op op, int dir, const SliceLists *slices, PrState *st, 
       *iters_out = h.iters;
       *resid_out = h.resid_last;
       if (scale_out) *scale_out = h.scale;
+      if (offset_out) *offset_out = h.offset;
       g->prof.add_bytes(kname, bytes_per_sweep * h.iters);
       return GG_OK;
     }
@@ -615,7 +730,7 @@ int gg_pagerank(gg_graph *g, float damping, const float *teleport, double tol_l1
   GG_HIP(fill_async<unsigned char>(reinterpret_cast<unsigned char *>(st), 0, sizeof(PrState), s));
   hipLaunchKernelGGL(k_pr_init, dim3(grid_for(n, kRowBlock, 4096)), dim3(kRowBlock), 0, s, r0,
                      weighted ? nullptr : x0, tele, g->pr[0].as<float>(), n, st, 0, (const float *)nullptr);
-  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(1), 0, s, st, 0);
+  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(kWave), 0, s, st, 0);
   GG_HIP(hipGetLastError());
   PrForwardOp op{};
   op.off = g->dg.column_offsets;
@@ -684,7 +799,6 @@ int gg_pagerank_adjoint(gg_graph *g, float damping, const float *rank, const flo
   GG_TRY(ensure_bins(g, 1));
   GG_TRY(ensure_transition(g));
   GG_TRY(g->batch[0].ensure(8 * (size_t)n));  // lambda[2]
-  GG_TRY(g->batch[1].ensure(4 * (size_t)n));  // rowsum
   GG_TRY(g->batch[2].ensure(sizeof(PrState)));
   const float *d_rank = nullptr, *d_c = nullptr;
   if (g->reordered) {
@@ -707,7 +821,7 @@ int gg_pagerank_adjoint(gg_graph *g, float damping, const float *rank, const flo
   GG_HIP(fill_async<unsigned char>(reinterpret_cast<unsigned char *>(st), 0, sizeof(PrState), s));
   hipLaunchKernelGGL(k_pr_init, dim3(grid_for(n, kRowBlock, 4096)), dim3(kRowBlock), 0, s, l0, (float *)nullptr,
                      (const float *)nullptr, g->pr[0].as<float>(), n, st, 1, d_c);
-  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(1), 0, s, st, 1);
+  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(kWave), 0, s, st, 1);
   GG_HIP(hipGetLastError());
   PrAdjointOp op{};
   op.off = g->dg.row_offsets;
@@ -717,11 +831,10 @@ int gg_pagerank_adjoint(gg_graph *g, float damping, const float *rank, const flo
   op.lam[0] = l0;
   op.lam[1] = l1;
   op.c = d_c;
-  op.rowsum = g->batch[1].as<float>();
   op.d = damping;
   op.inv_n = 1.0 / (double)n;
   op.st = st;
-  const double per_sweep = weighted ? 24.0 * n + 12.0 * m : 24.0 * n + 8.0 * m;
+  const double per_sweep = weighted ? 20.0 * n + 12.0 * m : 20.0 * n + 8.0 * m;
   SliceLists L{};
   const bool sliced = use_slices(g);
   if (sliced) {
@@ -730,10 +843,14 @@ int gg_pagerank_adjoint(gg_graph *g, float damping, const float *rank, const flo
     op.pcsr = weighted ? g->sl_val[1].as<float>() : nullptr;
   }
   int32_t iters = 0;
-  double resid = 0, scale = 1.0;  // scale = ||c||_1 (1 when c = 0)
+  double resid = 0, scale = 1.0, offset = 0.0;  // scale = ||c||_1 (1 when c = 0)
   GG_TRY(iterate(g, op, 1, sliced ? &L : nullptr, st, tol_l1, max_iter, "pagerank.adjoint_sweep", per_sweep, &iters,
-                 &resid, &scale));
-  const float *lam = (iters & 1) ? l1 : l0;
+                 &resid, &scale, &offset));
+  float *lam = (iters & 1) ? l1 : l0;
+  if (offset != 0.0) {
+    hipLaunchKernelGGL(k_add_offset, dim3(grid_for(n, 256, 8192)), dim3(256), 0, s, lam, st, n);
+    GG_HIP(hipGetLastError());
+  }
   // Gradients.
   float *gw = nullptr, *gt = nullptr;
   if (grad_w) {

@@ -390,3 +390,50 @@ def test_segmented_sweep_tile_shapes(gpu_available, weighted):
             np.testing.assert_array_equal(r2, r)
             np.testing.assert_array_equal(gw2, gw)
             np.testing.assert_array_equal(gt2, gt)
+
+
+@pytest.mark.parametrize("kind", ["one_edge", "cycle", "star", "two_components", "many_pairs", "rmat"])
+@pytest.mark.parametrize("loss", ["normal", "onehot", "ones", "zero"])
+def test_adjoint_constant_shift(gpu_available, kind, loss):
+    """The adjoint's sweeps remove the constant part of the error: the result
+    is still the FP64 adjoint, on graphs where the shift helps (rmat) and where
+    it cannot (several closed components, cycles: |lambda_2| = 1).  P has row
+    sums 1, so |e|_max <= d / (1 - d) |R|_max with |R|_max <= tol ||c||_1, plus
+    FP32 rounding of lambda amplified by 1 / (1 - d).  A plain sweep shrinks
+    |R|_max by d, so the run ends by the sweep where n d^k |R_0|_max reaches
+    tol ||c||_1, later by at most the 16 sweeps the shift is tried for."""
+    d, tol = 0.85, 2e-7
+    rng = np.random.default_rng(61)
+    if kind == "one_edge":
+        c = csr_from_edges(2, [0], [1])
+    elif kind == "cycle":
+        c = csr_from_edges(1025, np.arange(1025), (np.arange(1025) + 1) % 1025)
+    elif kind == "star":
+        c = csr_from_edges(1500, np.arange(1, 1500), np.zeros(1499))
+    elif kind == "two_components":
+        a = gg.gen_erdos_renyi(700, 3000, 5)
+        src = np.repeat(np.arange(a.n), a.degrees())
+        c = csr_from_edges(1401, np.concatenate([src, src + 701]), np.concatenate([a.col_indices, a.col_indices + 701]))
+    elif kind == "many_pairs":
+        a = gg.gen_rmat(11, 8, undirected=False, seed=62)
+        src = np.repeat(np.arange(a.n), a.degrees())
+        lo = a.n + 2 * np.arange(40)
+        c = csr_from_edges(a.n + 80, np.concatenate([src, lo, lo + 1]), np.concatenate([a.col_indices, lo + 1, lo]))
+    else:
+        c = gg.gen_rmat(12, 16, undirected=False, seed=63)
+    w = (rng.integers(1, 1 << 24, c.m) / 2.0**24).astype(np.float32)
+    c = gg.CSR(c.row_offsets, c.col_indices, w)
+    cv = {"normal": rng.standard_normal(c.n), "onehot": np.eye(1, c.n, c.n // 2)[0], "ones": np.ones(c.n),
+          "zero": np.zeros(c.n)}[loss].astype(np.float32).astype(np.float64)
+    r64, _, _ = oracle.pagerank_f64(c.row_offsets, c.col_indices, p=normalised_p32(c), tol=1e-15)
+    lam64, _, gt64, _ = oracle.pagerank_adjoint_f64(c.row_offsets, c.col_indices, w.astype(np.float64), r64, cv,
+                                                    tol=1e-15)
+    with gg.Graph(c, directed=True) as g:
+        _, gt, st = g.pagerank_adjoint(r64.astype(np.float32), cv.astype(np.float32), tol_l1=tol)
+    bound = d / (1 - d) * tol * np.abs(cv).sum() + 2.0**-22 / (1 - d) * np.abs(lam64).max()
+    assert np.abs(gt - gt64).max() <= (1 - d) * bound + 2.0**-23 * np.abs(gt64).max()
+    if loss != "zero":
+        plain = np.log(tol * np.abs(cv).sum() / (c.n * d * 2 * np.abs(cv).max())) / np.log(d)
+        assert st["residual"] <= tol * np.abs(cv).sum() and st["iterations"] <= np.ceil(plain) + 16
+    if kind == "rmat" and loss == "normal":
+        assert st["iterations"] <= 20
