@@ -1,4 +1,5 @@
-// Connected components by label propagation, device-driven (gg_cc default).
+// Connected components by label propagation, device-driven (gg_cc's default on
+// small graphs and under an iteration limit).
 //
 // Same semantics as the reference's CC program (Algorithms/CC/cc.h): every
 // vertex starts with its own id as label and active (cc.h:68-71,118-140); an
@@ -25,7 +26,11 @@
 //    swap) whose kernels read queue pointers, sizes and the direction from a
 //    device-side state block, so kIters iterations are captured once into a
 //    hipGraph and replayed until the frontier is empty, one host check per
-//    replay.  Bitmaps: a push clears, per frontier vertex, its word of the
+//    replay.  A frontier left after the first replay, with no iteration limit
+//    in the way, is finished by hooking (cc_hook_finish): the labels are a
+//    forest within the components by then (label[v] <= v is a vertex of v's
+//    component), and the rest costs a few passes instead of one per unit of
+//    diameter.  Bitmaps: a push clears, per frontier vertex, its word of the
 //    bitmap its frontier was deduplicated with (so that bitmap is clean when
 //    it becomes the next output bitmap); before a pull, and before the first
 //    push after a pull, the output bitmap is cleared whole.
@@ -311,9 +316,8 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
   const int grid = g->opt.expand_grid;
   g->prof.enabled = (flags & GG_INSTRUMENT) != 0;
 
-  ScopedEvents ev;
-  GG_HIP(ev.create());
-  hipEvent_t e0 = ev.e0, e1 = ev.e1;
+  hipEvent_t e0, e1;
+  GG_HIP(g->cc_ev.get(&e0, &e1));
   GG_HIP(hipEventRecord(e0, s));
   {
     TimedRegion t(g->prof, "cc.init");
@@ -349,6 +353,7 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
   };
   H h{};
   int rc = GG_OK;
+  bool hooked = false;
   for (;;) {
     {
       TimedRegion t(g->prof, "cc.labelprop");
@@ -364,12 +369,23 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
     }
     std::memcpy(&h, g->h_pinned, sizeof(H));
     if (h.done) break;
+    if (max_iter >= n) {  // a propagation never takes n iterations: the limit cannot end this run
+      GG_TRY(cc_hook_finish(g, label, false));
+      hooked = true;
+      break;
+    }
   }
   GG_TRY(rc);
   GG_HIP(hipEventRecord(e1, s));
   GG_HIP(hipEventSynchronize(e1));
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, e0, e1);
+  int64_t rest = 0;
+  if (hooked) {
+    GG_TRY(read_counters(g, 33));
+    rest = g->h64()[32];
+    g->prof.add_bytes("cc.rest", 8.0 * (double)rest + 8.0 * n);
+  }
   const double F = (double)h.frontier_total;
   const double bytes = 12.0 * n + words * 8.0 + 16.0 * (double)h.push_frontier + 8.0 * (double)h.edges +
                        (double)h.pulls * (12.0 * n + n / 8.0) + 8.0 * (F - n);
@@ -377,12 +393,13 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
   finish_profile(g);
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
-    stats->iterations = h.iters;
+    stats->iterations = h.iters + (hooked ? 1 : 0);
     stats->pull_iterations = h.pulls;
-    stats->edges_inspected = (int64_t)h.edges;
-    stats->alg_bytes = bytes;
+    stats->edges_inspected = (int64_t)h.edges + rest;
+    stats->alg_bytes = bytes + (hooked ? 16.0 * n + 8.0 * (double)rest : 0.0);
     stats->gpu_ms = ms;
-    GG_TRY(reach_stats(g, label, INT32_MIN, stats));
+    stats->reached_vertices = n;  // every vertex has a label
+    stats->reached_edges = g->m;
   }
   if (flags & GG_OUT_DEVICE) return GG_OK;
   return copy_out(g, label_out, label, 4 * (size_t)n, flags);

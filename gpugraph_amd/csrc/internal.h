@@ -306,7 +306,7 @@ struct gg_graph {
 
   // Device-driven BFS / SSSP loops: captured launch sequences and their
   // device-side loop state.
-  gg::RunEvents bfs_ev, sssp_ev;
+  gg::RunEvents bfs_ev, sssp_ev, cc_ev;
   gg::CapturedLoop bfs_loop[2];  // general BFS loop, by the parity of its first level
   gg::CapturedLoop sssp_loops[gg::kSsspReplayMax + 1];  // by iterations per replay
   gg::CapturedLoop sssp_resume;     // the iteration kernels after a stalled SSSP collect
@@ -387,6 +387,12 @@ int require_nonnegative_weights(gg_graph *g, const char *what);
 // instance-major (num x n) to host or device memory per flags; statistics
 // added to *acc.
 int batch_bfs(gg_graph *g, const int32_t *sources, int32_t num, int32_t *depth_out, uint32_t flags, gg_stats *acc);
+// Connected components by sampled hooking (cc_hook.hip); cc_hook_finish does
+// its second half: parent[] a forest within the components (parent[x] <= x)
+// in, labels out, enqueued on g->stream (rest edges in counter 32); linked:
+// as cc_hooking's first half leaves it.
+int cc_hooking(gg_graph *g, int32_t *label, uint32_t flags, gg_stats *stats);
+int cc_hook_finish(gg_graph *g, int32_t *parent, bool linked);
 // Symmetry / value-symmetry check of an undirected graph (sets mirror_ok,
 // values_asymmetric); GG_ERR_INVALID when the CSR is provably not symmetric.
 int check_undirected(gg_graph *g);

@@ -285,7 +285,7 @@ int reorder_out_cc(gg_graph *g, const int32_t *label, int32_t *dst, uint32_t fla
   if (!dst) return GG_OK;
   const int32_t n = g->n;
   hipStream_t s = g->stream;
-  DevBuf minold;
+  DevBuf &minold = g->re_out[1];  // kept with the graph: allocating it took most of the call
   GG_TRY(minold.ensure(4 * (size_t)n));
   GG_HIP(fill_async<int32_t>(minold.as<int32_t>(), INT_MAX, n, s));
   hipLaunchKernelGGL(k_cc_min_old, dim3(grid_for(n, 256, 16384)), dim3(256), 0, s, label, g->re_order.as<int32_t>(),

@@ -178,10 +178,12 @@ int gg_sssp(gg_graph *g, int32_t src, int32_t *dist, uint32_t flags,
 
 /* Connected-component labels = min vertex id of the component.  Replaces
  * EnactIterativeSearch with Program = cc (Algorithms/CC/cc.h:32-349; driver
- * cc.cu:291-292).  Default: the program's label propagation as a
- * device-driven loop (hipGraph replays, one host check per 16 iterations);
- * GG_CC_GAS: the same program through the generic GAS path; GG_CC_HOOK:
- * hooking + pointer jumping.  Undirected graphs. */
+ * cc.cu:291-292).  Default: below 2^17 vertices the program's label
+ * propagation as a device-driven loop (hipGraph replays), ended by hooking
+ * when 16 iterations have not been enough; from there on hooking, with
+ * stats->iterations its passes; with iter_num < n label propagation
+ * throughout.  GG_CC_GAS: the program through the generic GAS path;
+ * GG_CC_HOOK: hooking + pointer jumping at every size.  Undirected graphs. */
 int gg_cc(gg_graph *g, int32_t *label, uint32_t flags, gg_stats *stats);
 
 /* The reference's PageRank program (Algorithms/PageRank/PageRank.h:33-409):
