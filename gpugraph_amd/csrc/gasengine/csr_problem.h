@@ -9,6 +9,7 @@
 //                         reference's EDGE_FRONTIERS queues are 1.5*m each)
 //   dedup[2][ceil(n/32)]  bitmaps deduplicating the next frontier, alternated
 //                         per iteration and cleared word-wise by the consumer
+//   marks[n] (byte)       next frontier of an LBS expansion, before it is listed
 //   changed[n] (char), gather_tmp[n] (GatherType)
 //   scan_local[n], partials[ceil(n/1024)], LbsInfo, sizes[2], counters[8]
 #pragma once
@@ -46,6 +47,7 @@ struct Workspace {
   size_t gather_bytes = 0;
   int32_t *frontier[2] = {nullptr, nullptr};
   uint32_t *dedup[2] = {nullptr, nullptr};
+  uint8_t *marks = nullptr;  // words(n) * 32 bytes
   char *changed = nullptr;
   void *gather_tmp = nullptr;
   int32_t *scan_local = nullptr;
@@ -81,6 +83,7 @@ struct Workspace {
     GAS_RETURN_IF(hipMalloc(&frontier[1], nn * 4));
     GAS_RETURN_IF(hipMalloc(&dedup[0], nw * 4));
     GAS_RETURN_IF(hipMalloc(&dedup[1], nw * 4));
+    GAS_RETURN_IF(hipMalloc(&marks, nw * 32));
     GAS_RETURN_IF(hipMalloc(&changed, nn));
     GAS_RETURN_IF(hipMalloc(&gather_tmp, nn * (gather_elem_bytes > 4 ? gather_elem_bytes : 4)));
     GAS_RETURN_IF(hipMalloc(&scan_local, nn * 4));
@@ -140,7 +143,7 @@ struct Workspace {
     ResetLoop();
     if (cap_stream) (void)hipStreamDestroy(cap_stream);
     cap_stream = nullptr;
-    void *ps[] = {changed, gather_tmp, scan_local, partials, parts, info, sizes, counters, preds, ctl, gcarry,
+    void *ps[] = {marks, changed, gather_tmp, scan_local, partials, parts, info, sizes, counters, preds, ctl, gcarry,
                   order_words};
     for (void *p : ps)
       if (p) (void)hipFree(p);
@@ -151,6 +154,7 @@ struct Workspace {
     order_words = nullptr;
     gcarry = nullptr;
     gcarry_bytes = 0;
+    marks = nullptr;
     changed = nullptr;
     gather_tmp = nullptr;
     scan_local = nullptr;
@@ -286,6 +290,7 @@ struct CsrProblem {
     GAS_RETURN_IF(fill_async<char>(ws.changed, (char)0, n, stream));
     GAS_RETURN_IF(fill_async<uint32_t>(ws.dedup[0], 0u, Workspace::words(n), stream));
     GAS_RETURN_IF(fill_async<uint32_t>(ws.dedup[1], 0u, Workspace::words(n), stream));
+    GAS_RETURN_IF(fill_async<uint32_t>((uint32_t *)ws.marks, 0u, 8 * (int64_t)Workspace::words(n), stream));
     GAS_RETURN_IF(fill_async<unsigned long long>(ws.counters, 0ull, 8, stream));
     return hipSuccess;
   }

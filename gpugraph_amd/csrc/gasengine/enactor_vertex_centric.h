@@ -155,9 +155,10 @@ k_gas_ctl(GasCtl *c, int32_t *sizes, int sel, const int32_t *__restrict__ fronti
   c->gather_size = nf;
 }
 
-// The next frontier listed in vertex order from the dedup bitmap that built
-// it: always after an LBS expansion (whose edges only mark the bitmap, so no
-// workgroup serialises on the queue's size counter), and after a tiered one
+// The next frontier listed in vertex order from the dedup bitmap: always after
+// an LBS expansion (whose edges only mark vertices, so no workgroup serialises
+// on the queue's size counter; byte marks become the bitmap's words here, and
+// are cleared), and after a tiered one
 // (which appends, in whatever order its waves finish) when the frontier has
 // at least min_size vertices; the next iteration then reads its vertex
 // state and rows in runs of consecutive vertices.  Each thread counts a run
@@ -171,7 +172,7 @@ k_gas_ctl(GasCtl *c, int32_t *sizes, int sel, const int32_t *__restrict__ fronti
 constexpr int kOrderStage = 8192;
 template <int DUMMY = 0>
 __global__ void __launch_bounds__(kOrderBlock)
-k_gas_order(GasCtl *__restrict__ c, const uint32_t *__restrict__ bits, int32_t words, int32_t per_thread,
+k_gas_order(GasCtl *__restrict__ c, uint32_t *bits, uint8_t *__restrict__ marks, int32_t words, int32_t per_thread,
             int32_t *__restrict__ next_size, int32_t min_size, int32_t *__restrict__ queue,
             uint64_t *__restrict__ status) {
   if (c->done || (c->lbs_size == 0 && *next_size < min_size)) return;
@@ -181,8 +182,22 @@ k_gas_order(GasCtl *__restrict__ c, const uint32_t *__restrict__ bits, int32_t w
   __shared__ int32_t s_scan[kOrderBlock / kWave + 1];
   const int64_t w0 = ((int64_t)b * kOrderBlock + threadIdx.x) * per_thread;
   int32_t cnt = 0;
-  for (int k = 0; k < per_thread; k++)
-    if (w0 + k < words) cnt += __popc(bits[w0 + k]);
+  if (marks && c->lbs_size > 0) {
+    for (int k = 0; k < per_thread && w0 + k < words; k++) {
+      uint4 *p = reinterpret_cast<uint4 *>(marks) + 2 * (w0 + k);
+      const uint4 a = p[0], b4 = p[1];
+      auto nibble = [](uint32_t x) { return (x | x >> 7 | x >> 14 | x >> 21) & 15u; };  // four 0/1 bytes
+      const uint32_t word = nibble(a.x) | nibble(a.y) << 4 | nibble(a.z) << 8 | nibble(a.w) << 12 |
+                            nibble(b4.x) << 16 | nibble(b4.y) << 20 | nibble(b4.z) << 24 | nibble(b4.w) << 28;
+      if (!word) continue;  // the bitmap's word is 0 already
+      bits[w0 + k] = word;
+      p[0] = p[1] = make_uint4(0u, 0u, 0u, 0u);
+      cnt += __popc(word);
+    }
+  } else {
+    for (int k = 0; k < per_thread; k++)
+      if (w0 + k < words) cnt += __popc(bits[w0 + k]);
+  }
   int32_t total;
   int32_t pos = block_exclusive_scan<kOrderBlock>(cnt, s_scan, &total);
   const bool last = b == G - 1;
@@ -299,6 +314,7 @@ class EnactorVertexCentric {
     st.do_post = Program::postApplyOverEdges() != NO_POST_APPLY_VERTICES;
     st.iter_ptr = &ws.ctl->iter;
     st.preds = CsrProblemT::kMarkPredecessors ? ws.preds : nullptr;
+    st.marks = st.preds || detail::marks_in_bitmap<Program>() ? nullptr : ws.marks;
     return st;
   }
 
@@ -383,8 +399,8 @@ class EnactorVertexCentric {
     }
     for (int p = 0; p < np; p++) {
       st.in_edges = passes[p];
-      // The LBS expansion only marks the next frontier in dedup_next
-      // (k_gas_order lists it); the tiered one appends it.
+      // The LBS expansion only marks the next frontier (k_gas_order lists
+      // it); the tiered one appends it.
       GasState<Program> st_lbs = st;
       st_lbs.append = 0;
       st.append = 1;
@@ -432,7 +448,7 @@ class EnactorVertexCentric {
       const int grid = grid_for(words, kOrderBlock, kOrderGridMax);
       const int32_t per_thread = (int32_t)(((int64_t)words + (int64_t)grid * kOrderBlock - 1) / ((int64_t)grid * kOrderBlock));
       tb("order");
-      hipLaunchKernelGGL(k_gas_order<>, dim3(grid), dim3(kOrderBlock), 0, s, c, st.dedup_next, words,
+      hipLaunchKernelGGL(k_gas_order<>, dim3(grid), dim3(kOrderBlock), 0, s, c, st.dedup_next, st.marks, words,
                          per_thread < 1 ? 1 : per_thread, sz_out, std::max<int32_t>(n / 64, 4096), f_out,
                          ws.order_words);
       te("order");

@@ -41,9 +41,11 @@
 //   using Loads = ...                    what one edge's loads produce
 //   Loads load(int32_t v, int32_t val, int32_t slot)   loads only, no effects
 //   bool  apply(int32_t v, Loads l, int32_t &out)      as edge(), given l
-//   void  emit(bool keep, int32_t out, int32_t *s_out, int32_t *s_nout)
-//         optional: what becomes of apply()'s result (whole-wave call;
-//         default: wave_append to the tile's output list)
+//   void  emit<N>(const bool (&keep)[N], const int32_t (&out)[N],
+//                 int32_t *s_out, int32_t *s_nout)
+//         optional: what becomes of apply()'s results for the thread's N
+//         edges of the tile (whole-wave call, after all N applies; default:
+//         wave_append to the tile's output list, edge by edge)
 #pragma once
 
 #include <type_traits>
@@ -61,13 +63,14 @@ template <class Op>
 struct StagedEdge<Op, decltype((void)sizeof(typename Op::Loads))> {
   static constexpr bool value = true;
 };
-// An op may route apply()'s results itself: void emit(bool keep, int32_t
-// out, int32_t *s_out, int32_t *s_nout), called by every lane of the wave
-// (the default appends kept values to the tile's output list).
+// An op may route apply()'s results itself (emit, called by every lane of the
+// wave; the default appends kept values to the tile's output list).
 template <class Op, class = void>
 struct EdgeEmit : std::false_type {};
 template <class Op>
-struct EdgeEmit<Op, std::void_t<decltype(std::declval<Op &>().emit(false, 0, (int32_t *)nullptr, (int32_t *)nullptr))>>
+struct EdgeEmit<Op, std::void_t<decltype(std::declval<Op &>().emit(std::declval<const bool (&)[1]>(),
+                                                                    std::declval<const int32_t (&)[1]>(),
+                                                                    (int32_t *)nullptr, (int32_t *)nullptr))>>
     : std::true_type {};
 template <class Op, bool = StagedEdge<Op>::value>
 struct StagedEdgeLoads {
@@ -274,17 +277,17 @@ k_lbs_expand(Op op, const int32_t *__restrict__ frontier, const int32_t *__restr
           sl[r] = s;
           pre[r] = op.load(s_vert[s], Op::kItemValues ? s_val[s] : 0, s_begin[s] + (j0 + k - s_offs[s]));
         }
+        bool keep[VT];
+        int32_t out[VT];
 #pragma unroll
         for (int r = 0; r < VT; r++) {
           const int32_t k = (int32_t)threadIdx.x + r * kExpandBlock;
-          bool keep = false;
-          int32_t out = 0;
-          if (k < ne) keep = op.apply(s_vert[sl[r]], pre[r], out);
-          if constexpr (EdgeEmit<Op>::value)
-            op.emit(keep, out, s_out, &s_nout);
-          else
-            wave_append(keep, out, s_out, &s_nout);
+          keep[r] = false;
+          out[r] = 0;
+          if (k < ne) keep[r] = op.apply(s_vert[sl[r]], pre[r], out[r]);
+          if constexpr (!EdgeEmit<Op>::value) wave_append(keep[r], out[r], s_out, &s_nout);
         }
+        if constexpr (EdgeEmit<Op>::value) op.emit(keep, out, s_out, &s_nout);
       }
     } else {
       for (int32_t base = 0; base < ne; base += kExpandBlock) {

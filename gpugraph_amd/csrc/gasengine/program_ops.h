@@ -79,6 +79,13 @@ __device__ __forceinline__ void call_contract(int iteration, int &v, VT<P> &vl, 
     f(0, iteration, bitmap, v, vl, el, tmp, misc);  // 8-arg form: (rank_id, iteration, bitmap, ...)
 }
 
+// An 8-argument contract is handed the next frontier's bitmap: marks then go
+// there, where it can see them.
+template <class P>
+constexpr bool marks_in_bitmap() {
+  return arity<typename P::contract>() != 6;
+}
+
 template <class P, class = void>
 struct has_gather_vertex : std::false_type {};
 template <class P>
@@ -130,7 +137,8 @@ struct GasState {
   int do_post;
   const int32_t *iter_ptr;  // device-driven loops: the iteration number lives here (GasCtl::iter)
   int32_t *preds;           // MARK_PREDECESSORS: discovering vertex per vertex, else NULL
-  int append;               // 0: the next frontier is only marked in dedup_next (k_gas_order lists it)
+  int append;               // 0: the next frontier is only marked (k_gas_order lists it)
+  uint8_t *marks;           // a byte per vertex for those marks, or NULL: marked in dedup_next
 
   __device__ __forceinline__ int iter() const { return iter_ptr ? *iter_ptr : iteration; }
 };
@@ -193,8 +201,8 @@ struct ProgramOp {
                                    reinterpret_cast<unsigned char *>(s.dedup_next));
     if (frontier == -1) return false;
     if (!s.append && !s.preds) {
-      // Only marked (k_gas_order lists the next frontier from the bitmap):
-      // the caller sets the bit (emit), a whole wave's marks together.
+      // Only marked (k_gas_order lists the next frontier from the marks): the
+      // caller does it (emit), a whole wave's marks together.
       out = frontier;
       return true;
     }
@@ -205,19 +213,41 @@ struct ProgramOp {
     return true;
   }
 
-  // What k_lbs_expand does with apply()'s result, on every lane of the wave.
-  __device__ __forceinline__ void emit(bool keep, int32_t out, int32_t *s_out, int32_t *s_nout) {
-    if (!s.append && !s.preds)
-      wave_mark(keep, out, s.dedup_next);
-    else
-      wave_append(keep, out, s_out, s_nout);
+  // What k_lbs_expand does with apply()'s results, on every lane of the wave.
+  // A mark is a byte store, without an atomic: all writers store the same
+  // value and the stores combine in the L2s.  Bits took an atomicOr past the
+  // L2 for every mark whose word had not been seen set yet, which for a
+  // frontier of most vertices was most of the launch (PageRank program, 0.5M
+  // vertices and 12M edges: 169 us per expansion, 32 with
+  // bytes).  The bytes of the thread's N edges are read first, together:
+  // marks already seen end there.
+  template <int N>
+  __device__ __forceinline__ void emit(const bool (&keep)[N], const int32_t (&out)[N], int32_t *s_out,
+                                       int32_t *s_nout) {
+    if (!s.append && !s.preds && s.marks) {
+      uint8_t seen[N];
+#pragma unroll
+      for (int r = 0; r < N; r++) seen[r] = keep[r] ? s.marks[out[r]] : 1;
+#pragma unroll
+      for (int r = 0; r < N; r++)
+        if (!seen[r]) s.marks[out[r]] = 1;
+    } else if (!s.append && !s.preds) {
+#pragma unroll
+      for (int r = 0; r < N; r++) wave_mark(keep[r], out[r], s.dedup_next);
+    } else {
+#pragma unroll
+      for (int r = 0; r < N; r++) wave_append(keep[r], out[r], s_out, s_nout);
+    }
   }
 
   __device__ __forceinline__ bool edge(int32_t v, int32_t val, int32_t slot, int32_t &out) {
     int32_t o = 0;
     const bool keep = apply(v, load(v, val, slot), o);
     if (keep && !s.append && !s.preds) {
-      bit_test_and_set(s.dedup_next, o);
+      if (s.marks)
+        s.marks[o] = 1;
+      else
+        bit_test_and_set(s.dedup_next, o);
       return false;
     }
     out = o;
