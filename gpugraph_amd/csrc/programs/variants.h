@@ -29,8 +29,13 @@ struct cc_weak : cc {
 };
 
 namespace pagerank_detail {
-static __global__ void k_add_in_degree(const int *__restrict__ co, int *__restrict__ deg, int n) {
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) deg[v] += co[v + 1] - co[v];
+static __global__ void k_add_in_degree(const int *__restrict__ co, int *__restrict__ deg, float *__restrict__ share,
+                                       int n) {
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
+    const int d = deg[v] + co[v + 1] - co[v];
+    deg[v] = d;
+    share[v] = 0.15f / (float)d;
+  }
 }
 }  // namespace pagerank_detail
 
@@ -43,7 +48,8 @@ struct pagerank_all : pagerank {
                          d_row_indices, d_edge_values, vertex_list, edge_list, d_frontier_keys, d_frontier_values);
     if (nodes > 0)
       hipLaunchKernelGGL(pagerank_detail::k_add_in_degree, dim3(GASengine::grid_for(nodes, 256)), dim3(256), 0,
-                         GASengine::engine_stream(), d_column_offsets, vertex_list.d_num_out_edge, nodes);
+                         GASengine::engine_stream(), d_column_offsets, vertex_list.d_num_out_edge, vertex_list.d_share,
+                         nodes);
   }
   static GatherEdges gatherOverEdges() { return GATHER_ALL_EDGES; }
   static ExpandEdges expandOverEdges() { return EXPAND_ALL_EDGES; }
