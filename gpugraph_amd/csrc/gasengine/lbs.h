@@ -277,17 +277,29 @@ k_lbs_expand(Op op, const int32_t *__restrict__ frontier, const int32_t *__restr
           sl[r] = s;
           pre[r] = op.load(s_vert[s], Op::kItemValues ? s_val[s] : 0, s_begin[s] + (j0 + k - s_offs[s]));
         }
-        bool keep[VT];
-        int32_t out[VT];
+        if constexpr (EdgeEmit<Op>::value) {
+          bool keep[VT];
+          int32_t out[VT];
 #pragma unroll
-        for (int r = 0; r < VT; r++) {
-          const int32_t k = (int32_t)threadIdx.x + r * kExpandBlock;
-          keep[r] = false;
-          out[r] = 0;
-          if (k < ne) keep[r] = op.apply(s_vert[sl[r]], pre[r], out[r]);
-          if constexpr (!EdgeEmit<Op>::value) wave_append(keep[r], out[r], s_out, &s_nout);
+          for (int r = 0; r < VT; r++) {
+            const int32_t k = (int32_t)threadIdx.x + r * kExpandBlock;
+            keep[r] = false;
+            out[r] = 0;
+            if (k < ne) keep[r] = op.apply(s_vert[sl[r]], pre[r], out[r]);
+          }
+          op.emit(keep, out, s_out, &s_nout);
+        } else {
+          // One edge's result at a time: holding the VT results to the end
+          // made the SSSP push 9% slower.
+#pragma unroll
+          for (int r = 0; r < VT; r++) {
+            const int32_t k = (int32_t)threadIdx.x + r * kExpandBlock;
+            bool keep = false;
+            int32_t out = 0;
+            if (k < ne) keep = op.apply(s_vert[sl[r]], pre[r], out);
+            wave_append(keep, out, s_out, &s_nout);
+          }
         }
-        if constexpr (EdgeEmit<Op>::value) op.emit(keep, out, s_out, &s_nout);
       }
     } else {
       for (int32_t base = 0; base < ne; base += kExpandBlock) {
