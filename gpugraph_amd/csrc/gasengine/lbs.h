@@ -614,6 +614,7 @@ k_pull_staged(Op op, const int32_t *__restrict__ offs, int32_t n, int64_t m, con
   __shared__ int32_t s_state[TILE + 1];
   __shared__ int32_t s_slot[TILE];
   const int tid = threadIdx.x;
+  const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~(kWave - 1));
   const int64_t path = (int64_t)n + m;
   const int64_t G = gridDim.x;
   typename Op::Edge ed[VT];
@@ -635,8 +636,12 @@ k_pull_staged(Op op, const int32_t *__restrict__ offs, int32_t n, int64_t m, con
 #pragma unroll
       for (int r = 0; r < VT; r++) ed[r] = op.load_edge(jj0 + min(tid + r * kExpandBlock, nne - 1));
     }
+    // Only the waves that have a vertex of the tile: a tile of long rows holds
+    // few (about 60 at 16 edges a row), and loads of clamped slots took as many
+    // issue slots as the edges.
 #pragma unroll
     for (int q = 0; q < Q; q++) {
+      if (q * kExpandBlock + wave0 > nni + 1) break;
       const int32_t k = min(tid + q * kExpandBlock, nni + 1);
       const int32_t i = p0 - 1 + k;  // <= p1 <= n: offs has n + 1 entries
       ov[q] = i < 0 ? 0 : offs[i];
