@@ -437,3 +437,34 @@ def test_adjoint_constant_shift(gpu_available, kind, loss):
         assert st["residual"] <= tol * np.abs(cv).sum() and st["iterations"] <= np.ceil(plain) + 16
     if kind == "rmat" and loss == "normal":
         assert st["iterations"] <= 20
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_adjoint_gradient_row_lengths(gpu_available, weighted):
+    """The gradient pass over rows at the edges of its kernels: one thread up to
+    32 edges, a wave up to 4096 (256 edges a step), a 1024-thread workgroup
+    beyond (4096 a step), against the FP64 adjoint.  The relative L2 error of
+    the edge gradient stays below 1e-4, the bound of the other adjoint tests."""
+    lengths = [0, 1, 31, 32, 33, 255, 256, 257, 4095, 4096, 4097, 8191, 8192, 8193]
+    n = 9000
+    rng = np.random.default_rng(65)
+    src = np.concatenate([np.repeat(np.arange(len(lengths)), lengths), np.repeat(np.arange(20, n), 3)])
+    dst = np.concatenate([rng.choice(n, k, replace=False) for k in lengths if k] + [rng.integers(0, n, 3 * (n - 20))])
+    c = csr_from_edges(n, src, dst)
+    if weighted:
+        c = gg.CSR(c.row_offsets, c.col_indices, (rng.integers(1, 1 << 24, c.m) / 2.0**24).astype(np.float32))
+    cv = rng.standard_normal(n)
+    p = normalised_p32(c) if weighted else None
+    r64, _, _ = oracle.pagerank_f64(c.row_offsets, c.col_indices, p=p, tol=1e-15)
+    w64 = c.values.astype(np.float64) if weighted else np.ones(c.m)
+    lam, gw64, _, _ = oracle.pagerank_adjoint_f64(c.row_offsets, c.col_indices, w64, r64, cv, tol=1e-15)
+    rows = np.repeat(np.arange(n), c.degrees())
+    if not weighted:  # dL/dP_uv = d r_u lambda_v
+        gw64 = 0.85 * r64[rows] * lam[c.col_indices]
+    with gg.Graph(c, directed=True) as g:
+        gw, _, _ = g.pagerank_adjoint(r64.astype(np.float32), cv.astype(np.float32), tol_l1=2e-7)
+    for i, k in enumerate(lengths):
+        row = rows == i
+        if k > 1:  # a single edge's weight does not matter: its gradient is 0 but for rounding
+            assert np.linalg.norm(gw[row] - gw64[row]) / np.linalg.norm(gw64[row]) < 1e-4, k
+    assert np.linalg.norm(gw - gw64) / np.linalg.norm(gw64) < 1e-4
