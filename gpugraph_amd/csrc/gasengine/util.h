@@ -89,41 +89,48 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-// Inclusive scan across the wave.
+// v moved by a DPP pattern, 0 where the source lane is outside its row or the
+// row is masked off.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int32_t dpp_or_zero(int32_t v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+
+// Inclusive scan across the wave: within rows of 16 lanes by row shifts, then
+// lane 15's and lane 31's sums broadcast to the rows above them.  All lanes
+// take part.  (Shuffles go through the LDS unit, six of them in a chain.)
 __device__ __forceinline__ int32_t wave_inclusive_scan(int32_t v) {
-  const int l = lane_id();
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    int32_t t = __shfl_up(v, off);
-    if (l >= off) v += t;
-  }
+  v += dpp_or_zero<0x111, 0xf>(v);  // row_shr:1
+  v += dpp_or_zero<0x112, 0xf>(v);  // row_shr:2
+  v += dpp_or_zero<0x114, 0xf>(v);  // row_shr:4
+  v += dpp_or_zero<0x118, 0xf>(v);  // row_shr:8
+  v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15 to rows 1 and 3
+  v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31 to rows 2 and 3
   return v;
 }
 
 // Exclusive scan over a workgroup of BLOCK threads.  `smem` needs
 // BLOCK/64 + 1 ints.  Returns the exclusive prefix; *total gets the sum.
+// Every thread adds up the wave totals itself: one barrier less than having
+// one thread scan them, which in the short launches of an iteration (collect,
+// count, order) was a good part of the time.
 template <int BLOCK>
 __device__ __forceinline__ int32_t block_exclusive_scan(int32_t v, int32_t *smem, int32_t *total) {
   constexpr int W = BLOCK / kWave;
-  const int wid = threadIdx.x / kWave, l = lane_id();
-  int32_t inc = wave_inclusive_scan(v);
-  if (l == kWave - 1) smem[wid] = inc;
+  const int wid = threadIdx.x / kWave;
+  const int32_t inc = wave_inclusive_scan(v);
+  if (lane_id() == kWave - 1) smem[wid] = inc;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t run = 0;
+  int32_t before = 0, sum = 0;
 #pragma unroll
-    for (int w = 0; w < W; w++) {
-      int32_t t = smem[w];
-      smem[w] = run;
-      run += t;
-    }
-    smem[W] = run;
+  for (int w = 0; w < W; w++) {
+    const int32_t t = smem[w];
+    before += w < wid ? t : 0;
+    sum += t;
   }
+  *total = sum;
   __syncthreads();
-  int32_t excl = smem[wid] + inc - v;
-  *total = smem[W];
-  __syncthreads();
-  return excl;
+  return before + inc - v;
 }
 
 // Workgroup sum of 64-bit values; result valid in every thread.
