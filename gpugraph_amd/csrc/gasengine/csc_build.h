@@ -80,7 +80,7 @@ __global__ void k_column_offsets(const int32_t *__restrict__ keys, int64_t m, in
 }
 
 // Transpose a validated device CSR into caller-provided co[n+1], ri[m],
-// eid[m] on stream s (synchronises s; temporaries are freed before return).
+// eid[m] on stream s (synchronises s).
 // Returns the first HIP error, allocations included.
 inline hipError_t device_csr_to_csc(int32_t n, int64_t m, const int32_t *ro, const int32_t *col, int32_t *co,
                                     int32_t *ri, int32_t *eid, hipStream_t s) {
@@ -92,9 +92,10 @@ inline hipError_t device_csr_to_csc(int32_t n, int64_t m, const int32_t *ro, con
   int32_t *keys_out = nullptr, *ids = nullptr, *rows = nullptr;
   int end_bit = 1;
   while (end_bit < 31 && ((int64_t)1 << end_bit) < n) end_bit++;
-  hipError_t e = hipMalloc((void **)&keys_out, 4 * (size_t)m);
-  if (e == hipSuccess) e = hipMalloc((void **)&ids, 4 * (size_t)m);
-  if (e == hipSuccess) e = hipMalloc((void **)&rows, 4 * (size_t)m);
+  PoolScratch scratch;
+  hipError_t e = scratch.alloc(&keys_out, 4 * (size_t)m);
+  if (e == hipSuccess) e = scratch.alloc(&ids, 4 * (size_t)m);
+  if (e == hipSuccess) e = scratch.alloc(&rows, 4 * (size_t)m);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_iota<0>, dim3(grid_for(m, 256, 16384)), dim3(256), 0, s, ids, m);
     hipLaunchKernelGGL(k_edge_rows<0>, dim3(grid_for((int64_t)n * kWave, 256, 16384)), dim3(256), 0, s, ro, n, rows);
@@ -108,10 +109,8 @@ inline hipError_t device_csr_to_csc(int32_t n, int64_t m, const int32_t *ro, con
     e = hipGetLastError();
   }
   const hipError_t sy = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = sy;
-  for (void *p : {(void *)keys_out, (void *)ids, (void *)rows})
-    if (p) (void)hipFree(p);
-  return e;
+  if (sy == hipSuccess) scratch.released();
+  return e == hipSuccess ? sy : e;
 }
 
 }  // namespace GASengine

@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pool.h"
 #include "util.h"
 
 namespace GASengine {
@@ -193,10 +194,11 @@ hipError_t radix_sort_pairs(const K *keys_in, K *keys_out, const V *vals_in, V *
   K *kt = nullptr;
   V *vt = nullptr;
   int32_t *hist = nullptr, *totals = nullptr;
-  hipError_t e = hipMalloc((void **)&kt, sizeof(K) * (size_t)count);
-  if (e == hipSuccess) e = hipMalloc((void **)&vt, sizeof(V) * (size_t)count);
-  if (e == hipSuccess) e = hipMalloc((void **)&hist, sizeof(int32_t) * (size_t)cells);
-  if (e == hipSuccess) e = hipMalloc((void **)&totals, sizeof(int32_t) * (size_t)scan_totals_entries(cells));
+  PoolScratch scratch;
+  hipError_t e = scratch.alloc(&kt, sizeof(K) * (size_t)count);
+  if (e == hipSuccess) e = scratch.alloc(&vt, sizeof(V) * (size_t)count);
+  if (e == hipSuccess) e = scratch.alloc(&hist, sizeof(int32_t) * (size_t)cells);
+  if (e == hipSuccess) e = scratch.alloc(&totals, sizeof(int32_t) * (size_t)scan_totals_entries(cells));
   if (e == hipSuccess) {
     const int grid = (int)(tiles < kSortGridMax ? tiles : kSortGridMax);
     // The last pass lands in keys_out: with an odd number of passes the
@@ -222,10 +224,8 @@ hipError_t radix_sort_pairs(const K *keys_in, K *keys_out, const V *vals_in, V *
     }
   }
   const hipError_t sy = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = sy;
-  for (void *p : {(void *)kt, (void *)vt, (void *)hist, (void *)totals})
-    if (p) (void)hipFree(p);
-  return e;
+  if (sy == hipSuccess) scratch.released();
+  return e == hipSuccess ? sy : e;
 }
 
 }  // namespace GASengine

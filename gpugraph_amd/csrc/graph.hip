@@ -454,14 +454,21 @@ int gg_graph_create(int32_t n, int64_t m, const int32_t *row_offsets, const int3
   GG_HIP(hipHostMalloc((void **)&g->h_pinned, (GASengine::kCounterSlots + GASengine::kCounterWords) * sizeof(int64_t)));
   GG_HIP(hipHostGetDevicePointer((void **)&g->h_dev, g->h_pinned, 0));
 
-  const hipMemcpyKind kind = dev_in ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+  // Host arrays on the handle's own stream (the legacy stream would break a
+  // capture of another thread); device arrays on the legacy stream, after the
+  // work that wrote them.
+  auto load = [&](void *dst, const void *src, size_t bytes) -> hipError_t {
+    if (dev_in) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToDevice);
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g->stream);
+    return e != hipSuccess ? e : hipStreamSynchronize(g->stream);
+  };
   GG_TRY(g->ro.ensure(4 * ((size_t)n + 1)));
   GG_TRY(g->col.ensure(4 * (size_t)std::max<int64_t>(m, 1)));
-  GG_HIP(hipMemcpy(g->ro.p, row_offsets, 4 * ((size_t)n + 1), kind));
-  if (m) GG_HIP(hipMemcpy(g->col.p, col_indices, 4 * (size_t)m, kind));
+  GG_HIP(load(g->ro.p, row_offsets, 4 * ((size_t)n + 1)));
+  if (m) GG_HIP(load(g->col.p, col_indices, 4 * (size_t)m));
   if (value_dtype != GG_VALUES_NONE) {
     GG_TRY(g->val.ensure(4 * (size_t)std::max<int64_t>(m, 1)));
-    if (m) GG_HIP(hipMemcpy(g->val.p, values, 4 * (size_t)m, kind));
+    if (m) GG_HIP(load(g->val.p, values, 4 * (size_t)m));
   }
   // Validate the CSR on the device before any kernel indexes with it.
   {
@@ -523,7 +530,15 @@ int gg_graph_destroy(gg_graph *g) {
   g->prof.reset();
   if (g->h_pinned) (void)hipHostFree(g->h_pinned);
   if (g->own_stream && g->stream) (void)hipStreamDestroy(g->stream);
+  // The buffers go to the block pool once nothing can use them: hipFree of one
+  // (the counters, small) waits for the whole device, since callers may read
+  // the resident CSR on streams of their own, without disturbing a capture of
+  // another thread.
+  const bool waited = g->counters.p != nullptr;
+  g->counters.reset();
+  gg::t_device_idle = waited;
   delete g;
+  gg::t_device_idle = false;
   if (cur >= 0 && cur != dev) (void)hipSetDevice(cur);
   return GG_OK;
 }

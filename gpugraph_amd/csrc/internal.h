@@ -29,7 +29,12 @@ namespace gg {
     if (_rc != GG_OK) return _rc;  \
   } while (0)
 
-// Device buffer owned by a graph handle.
+// Set while gg_graph_destroy releases a handle's buffers, after it has waited
+// for the device: nothing can still use them, so they may go to the pool.
+inline thread_local bool t_device_idle = false;
+
+// Device buffer owned by a graph handle.  Taken from the block pool; given back
+// to it when the handle is destroyed, freed (waiting for the device) otherwise.
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
@@ -38,7 +43,10 @@ struct DevBuf {
   DevBuf &operator=(const DevBuf &) = delete;
   ~DevBuf() { reset(); }
   void reset() {
-    if (p) (void)hipFree(p);
+    if (p && t_device_idle)
+      GASengine::BlockPool::get().give(p, bytes);
+    else if (p)
+      (void)hipFree(p);
     p = nullptr;
     bytes = 0;
   }
@@ -47,12 +55,8 @@ struct DevBuf {
     if (want == 0) want = 4;
     if (bytes >= want) return GG_OK;
     reset();
-    hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess) {
-      p = nullptr;
-      return set_error(GG_ERR_OOM, "hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
-    }
-    bytes = want;
+    hipError_t e = GASengine::BlockPool::get().take(want, &p, &bytes);
+    if (e != hipSuccess) return set_error(GG_ERR_OOM, "hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
     return GG_OK;
   }
   template <class T>
