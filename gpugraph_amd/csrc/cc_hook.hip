@@ -25,8 +25,8 @@
 // a root is read again before its CAS: 2.4 -> 0.09 ms on an R-MAT), the others
 // by latency and launches: each moves about 8 n bytes, against 8 m for hooking
 // every edge.  Per call, against label propagation / hooking every edge:
-// 2048 x 2048 lattice (4.2M vertices, 10M edges) 12.1 / 0.66 -> 0.44 ms; R-MAT
-// of 1.5M vertices and 35M edges 0.90 -> 0.22 ms; of 4.2M vertices and 128M
+// 2048 x 2048 lattice (4.2M vertices, 10M edges) 12.4 / 0.66 -> 0.42 ms; R-MAT
+// of 1.5M vertices and 35M edges 0.92 -> 0.16-0.20 ms; of 4.2M vertices and 128M
 // edges 3.86 / 3.89 -> 0.27 ms, renumbered by degree 2.02 / 6.36 -> 0.32 ms;
 // path, band, star and pair graphs of 2M vertices 0.08-0.30 ms.
 //
