@@ -25,9 +25,9 @@
 //  * Device-driven loop: an iteration is a fixed launch sequence (push, pull,
 //    swap) whose kernels read queue pointers, sizes and the direction from a
 //    device-side state block, so kIters iterations are captured once into a
-//    hipGraph and replayed until the frontier is empty, one host check per
-//    replay.  A frontier left after the first replay, with no iteration limit
-//    in the way, is finished by hooking (cc_hook_finish): the labels are a
+//    hipGraph, kept on the handle, and replayed until the frontier is empty,
+//    one host check per replay.  A frontier left after the first replay, with
+//    no iteration limit in the way, is finished by hooking (cc_hook_finish): the labels are a
 //    forest within the components by then (label[v] <= v is a vertex of v's
 //    component), and the rest costs a few passes instead of one per unit of
 //    diameter.  Bitmaps: a push clears, per frontier vertex, its word of the
@@ -296,14 +296,11 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
   const int32_t n = g->n;
   const size_t words = ((size_t)n + 31) / 32;
   hipStream_t s = g->stream;
-  int32_t *label;
-  if (flags & GG_OUT_DEVICE) {
-    GG_CHECK_ARG(label_out, "label is NULL");
-    label = label_out;
-  } else {
-    GG_TRY(g->vtx[1].ensure(4 * (size_t)n));
-    label = g->vtx[1].as<int32_t>();
-  }
+  if (flags & GG_OUT_DEVICE) GG_CHECK_ARG(label_out, "label is NULL");
+  // The loop runs on the handle's own labels, copied out at the end: its
+  // capture then serves every output buffer.
+  GG_TRY(g->vtx[1].ensure(4 * (size_t)n));
+  int32_t *label = g->vtx[1].as<int32_t>();
   GG_TRY(g->frontier[0].ensure(4 * (size_t)n));
   GG_TRY(g->frontier[1].ensure(4 * (size_t)n));
   GG_TRY(g->bits[0].ensure(4 * words));
@@ -331,21 +328,42 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
   g->prof.add_bytes("cc.init", 12.0 * n + words * 8.0);
   const int32_t *parts = nullptr;
   GG_TRY(pull_partition(g, &parts));  // merge-path tiles over (vertices, adjacency), cached per graph
-  CcPullOp pull_op{g->dg.column_indices, label, st, 0ull};
-  ScopedGraph cg;
-  GG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-  for (int it = 0; it < kIters; it++) {
-    hipLaunchKernelGGL(k_lp_prep, dim3(grid_for((int64_t)words, kBlock, 1024)), dim3(kBlock), 0, s, st,
-                       (int32_t)words);
-    hipLaunchKernelGGL(k_lp_expand, dim3(grid), dim3(kBlock), 0, s, st, g->dg.row_offsets, g->dg.column_indices,
-                       label, g->opt.wave_degree);
-    hipLaunchKernelGGL((k_pull_staged<CcPullOp, int32_t>), dim3(grid), dim3(kExpandBlock), 0, s, pull_op,
-                       g->dg.row_offsets, n, g->m, parts, &st->pull_skip);
-    hipLaunchKernelGGL(k_lp_swap, dim3(1), dim3(1), 0, s, st, n, g->m, max_iter);
+  // kIters iterations captured once per handle and set of arguments.  A capture
+  // made and destroyed by every call cost about 100 us of it, and three times
+  // that where the next call began right after the last replay (capture,
+  // instantiation and destruction each 2-4 times slower then): 450-550 us a
+  // call on a 7020-vertex R-MAT with the labels left on the device, 300-330
+  // with host output; kept, 194 and 211.
+  const std::vector<uint64_t> key = {(uint64_t)label, (uint64_t)q0,   (uint64_t)q1,
+                                     (uint64_t)b0,    (uint64_t)b1,   (uint64_t)st,
+                                     (uint64_t)parts, (uint64_t)grid, (uint64_t)g->opt.wave_degree,
+                                     (uint64_t)max_iter};
+  CapturedLoop &loop = g->cc_loop;
+  if (!loop.exec || loop.key != key) {
+    loop.reset();
+    CcPullOp pull_op{g->dg.column_indices, label, st, 0ull};
+    hipGraph_t graph = nullptr;
+    GG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+    for (int it = 0; it < kIters; it++) {
+      hipLaunchKernelGGL(k_lp_prep, dim3(grid_for((int64_t)words, kBlock, 1024)), dim3(kBlock), 0, s, st,
+                         (int32_t)words);
+      hipLaunchKernelGGL(k_lp_expand, dim3(grid), dim3(kBlock), 0, s, st, g->dg.row_offsets, g->dg.column_indices,
+                         label, g->opt.wave_degree);
+      hipLaunchKernelGGL((k_pull_staged<CcPullOp, int32_t>), dim3(grid), dim3(kExpandBlock), 0, s, pull_op,
+                         g->dg.row_offsets, n, g->m, parts, &st->pull_skip);
+      hipLaunchKernelGGL(k_lp_swap, dim3(1), dim3(1), 0, s, st, n, g->m, max_iter);
+    }
+    const hipError_t cap = hipStreamEndCapture(s, &graph);
+    hipError_t inst = hipErrorUnknown;
+    if (cap == hipSuccess) inst = hipGraphInstantiate(&loop.exec, graph, nullptr, nullptr, 0);
+    if (graph) (void)hipGraphDestroy(graph);
+    if (inst != hipSuccess) {
+      loop.exec = nullptr;
+      return set_error(GG_ERR_HIP, "CC loop capture failed: %s / %s", hipGetErrorString(cap),
+                       hipGetErrorString(inst));
+    }
+    loop.key = key;
   }
-  hipError_t cap = hipStreamEndCapture(s, &cg.graph);
-  if (cap != hipSuccess) return set_error(GG_ERR_HIP, "graph capture failed: %s", hipGetErrorString(cap));
-  GG_HIP(hipGraphInstantiate(&cg.exec, cg.graph, nullptr, nullptr, 0));
   struct H {
     int32_t iters, done;
     unsigned long long edges, frontier_total, push_frontier;
@@ -357,7 +375,7 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
   for (;;) {
     {
       TimedRegion t(g->prof, "cc.labelprop");
-      if (hipGraphLaunch(cg.exec, s) != hipSuccess) {
+      if (hipGraphLaunch(loop.exec, s) != hipSuccess) {
         rc = set_error(GG_ERR_HIP, "graph launch failed");
         break;
       }
@@ -401,7 +419,6 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
     stats->reached_vertices = n;  // every vertex has a label
     stats->reached_edges = g->m;
   }
-  if (flags & GG_OUT_DEVICE) return GG_OK;
   return copy_out(g, label_out, label, 4 * (size_t)n, flags);
 }
 

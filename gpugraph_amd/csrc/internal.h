@@ -308,9 +308,10 @@ struct gg_graph {
   // Generic-program state kept across runs (one per program type).
   std::shared_ptr<void> prog_state[8];
 
-  // Device-driven BFS / SSSP loops: captured launch sequences and their
+  // Device-driven BFS / SSSP / CC loops: captured launch sequences and their
   // device-side loop state.
   gg::RunEvents bfs_ev, sssp_ev, cc_ev;
+  gg::CapturedLoop cc_loop;      // label propagation: one replay's iterations
   gg::CapturedLoop bfs_loop[2];  // general BFS loop, by the parity of its first level
   gg::CapturedLoop sssp_loops[gg::kSsspReplayMax + 1];  // by iterations per replay
   gg::CapturedLoop sssp_resume;     // the iteration kernels after a stalled SSSP collect
