@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -308,6 +309,47 @@ int check_undirected(gg_graph *g) {
   return GG_OK;
 }
 
+// Host array to the device, complete on return.  Not on the legacy stream,
+// where a copy breaks the capture of a loop that another thread's handle is
+// making, and not on the handle's own: the first copies of a new stream set up
+// its staging (0.45 ms; a 70773-vertex, 424k-edge graph loaded in 1.05 ms so,
+// 0.60 as here).  One stream per device, shared by all handles and kept.
+// Memory that the runtime knows (pinned, managed) may be the target of work
+// still in flight on any stream, which a copy on the legacy stream would have
+// waited for: the device is waited for instead, by hipFree, since
+// hipDeviceSynchronize breaks such captures too.
+static hipStream_t upload_stream(int device) {
+  constexpr int kDevices = 64;
+  static std::mutex mutex;
+  static hipStream_t streams[kDevices];
+  if (device < 0 || device >= kDevices) return nullptr;
+  std::lock_guard<std::mutex> lock(mutex);
+  if (!streams[device] && hipStreamCreateWithFlags(&streams[device], hipStreamNonBlocking) != hipSuccess)
+    streams[device] = nullptr;
+  return streams[device];
+}
+
+static hipError_t upload(gg_graph *g, void *dst, const void *src, size_t bytes) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, src) != hipSuccess) {
+    (void)hipGetLastError();  // memory the runtime does not know
+  } else if (at.type != hipMemoryTypeUnregistered) {
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, 4);
+    if (e == hipSuccess) e = hipFree(p);
+    if (e != hipSuccess) return e;
+  }
+  hipStream_t s = upload_stream(g->device);
+  if (!s) s = g->stream;
+  hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+  if (e != hipSuccess && s != g->stream) {  // the caller has reset the device since: the stream is gone
+    (void)hipGetLastError();
+    s = g->stream;
+    e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+  }
+  return e != hipSuccess ? e : hipStreamSynchronize(s);
+}
+
 int lbs_buffers(gg_graph *g, GASengine::LbsBuffers *b) {
   const size_t n = (size_t)g->n;
   GG_TRY(g->frontier[0].ensure(4 * n));
@@ -454,13 +496,9 @@ int gg_graph_create(int32_t n, int64_t m, const int32_t *row_offsets, const int3
   GG_HIP(hipHostMalloc((void **)&g->h_pinned, (GASengine::kCounterSlots + GASengine::kCounterWords) * sizeof(int64_t)));
   GG_HIP(hipHostGetDevicePointer((void **)&g->h_dev, g->h_pinned, 0));
 
-  // Host arrays on the handle's own stream (the legacy stream would break a
-  // capture of another thread); device arrays on the legacy stream, after the
-  // work that wrote them.
+  // Device arrays on the legacy stream, after the work that wrote them.
   auto load = [&](void *dst, const void *src, size_t bytes) -> hipError_t {
-    if (dev_in) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToDevice);
-    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g->stream);
-    return e != hipSuccess ? e : hipStreamSynchronize(g->stream);
+    return dev_in ? hipMemcpy(dst, src, bytes, hipMemcpyDeviceToDevice) : gg::upload(g, dst, src, bytes);
   };
   GG_TRY(g->ro.ensure(4 * ((size_t)n + 1)));
   GG_TRY(g->col.ensure(4 * (size_t)std::max<int64_t>(m, 1)));
