@@ -16,9 +16,11 @@
 //   2 link     every vertex hooks with its second neighbour, then flatten
 //   3 giant    the most frequent root among kSamples vertices
 //   4 rest     only the vertices outside that tree hook along their rows; an
-//              edge between it and them is seen from their side (the graph is
-//              symmetric), rows of kLongRow edges and more in chunks that the
-//              whole grid shares
+//              edge between it and them is seen from their side, which holds
+//              it as well where the handle's check found the mirror of every
+//              entry (rows that are not sorted are not checked: there every
+//              vertex hooks); rows of kLongRow edges and more in chunks that
+//              the whole grid shares
 //   5 labels   parent[v] = root
 // The link pass is bound by its chains of dependent loads and by atomics on
 // the roots that most trees join (a wave sends one hook per pair of roots, and
@@ -176,7 +178,9 @@ __device__ __forceinline__ int32_t walk_to_root(const int32_t *parent, int32_t x
 
 // The most frequent root of kSamples vertices spread over the ids (one
 // workgroup; every thread counts its own sample's root in LDS).
-__global__ void __launch_bounds__(kSamples) k_cc_giant(const int32_t *parent, int32_t n, CcCtl *ctl) {
+// mirrored = false: no tree is left out, whatever its size.
+__global__ void __launch_bounds__(kSamples)
+k_cc_giant(const int32_t *parent, int32_t n, bool mirrored, CcCtl *ctl) {
   __shared__ __align__(16) int32_t s_root[kSamples];
   __shared__ unsigned long long s_best;
   const int t = threadIdx.x;
@@ -194,13 +198,13 @@ __global__ void __launch_bounds__(kSamples) k_cc_giant(const int32_t *parent, in
   atomicMax(&s_best, ((unsigned long long)same << 32) | (uint32_t)r);
   __syncthreads();
   if (t == 0) {
-    ctl->giant = (int32_t)(uint32_t)s_best;
+    ctl->giant = mirrored ? (int32_t)(uint32_t)s_best : -1;
     ctl->chunks = 0;
   }
 }
 
-// Every edge of a vertex outside the giant tree is hooked from its side: a
-// vertex that joined the giant tree before its turn leaves its row out, and
+// Every edge of a vertex outside the giant tree (no such tree: -1) is hooked
+// from its side: a vertex that joined the giant tree before its turn leaves its row out, and
 // the far end of such an edge has either joined as well or hooks it itself.
 // linked: k_cc_init and k_cc_link have run, so a vertex has been joined with
 // its second neighbour, and with its first one where that is smaller.
@@ -290,7 +294,7 @@ int cc_hook_finish(gg_graph *g, int32_t *parent, bool linked) {
     TimedRegion t(g->prof, "cc.rest");
     GG_HIP(slot_resets_async(ctr, {{32, 0ull}}, s));
     hipLaunchKernelGGL(k_cc_flatten, grid, block, 0, s, parent, n);
-    hipLaunchKernelGGL(k_cc_giant, dim3(1), dim3(kSamples), 0, s, parent, n, ctl);
+    hipLaunchKernelGGL(k_cc_giant, dim3(1), dim3(kSamples), 0, s, parent, n, g->mirror_ok, ctl);
     hipLaunchKernelGGL(k_cc_rest, grid, block, 0, s, parent, ro, col, n, ctl, chunks, ctr + 32, linked);
     hipLaunchKernelGGL(k_cc_rest_chunks, dim3(512), block, 0, s, parent, ro, col, ctl, chunks);
     GG_HIP(hipGetLastError());

@@ -51,7 +51,8 @@ extern "C" {
 /* ---- graph flags ------------------------------------------------------- */
 #define GG_GRAPH_DIRECTED 1u    /* build the CSC (in-edges) on the device;
                                    otherwise the CSR must be symmetric and is
-                                   used as its own CSC */
+                                   used as its own CSC (checked at creation
+                                   where the rows are sorted) */
 #define GG_GRAPH_DEVICE_PTRS 2u /* inputs are device pointers on the current device */
 #define GG_GRAPH_REORDER 4u     /* store the graph renumbered by out-degree, highest first (locality
                                    of the random vertex gathers); every call still takes and
@@ -183,7 +184,9 @@ int gg_sssp(gg_graph *g, int32_t src, int32_t *dist, uint32_t flags,
  * when 16 iterations have not been enough; from there on hooking, with
  * stats->iterations its passes; with iter_num < n label propagation
  * throughout.  GG_CC_GAS: the program through the generic GAS path;
- * GG_CC_HOOK: hooking + pointer jumping at every size.  Undirected graphs. */
+ * GG_CC_HOOK: hooking + pointer jumping at every size.  Undirected graphs.
+ * Hooking joins the ends of every entry, also where rows are not sorted and
+ * an entry has no mirror. */
 int gg_cc(gg_graph *g, int32_t *label, uint32_t flags, gg_stats *stats);
 
 /* The reference's PageRank program (Algorithms/PageRank/PageRank.h:33-409):

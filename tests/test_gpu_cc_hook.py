@@ -77,3 +77,26 @@ def test_default_switch(gpu_available, name, n):
         lab, st = g.cc()
         assert st["iterations"] == 1
         assert np.all(lab >= exp) and (name == "pairs" or np.any(lab > exp))
+
+
+@pytest.mark.parametrize("n", [3000, (1 << 17) + 5])
+def test_unsorted_rows_without_mirrors(gpu_available, n):
+    """Rows that are not sorted cannot be checked for symmetry, so an edge may
+    be stored at one end only, here in the rows of the largest tree: hooking
+    still joins both ends."""
+    rng = np.random.default_rng(73)
+    big = 2 * n // 3
+    a, b = rng.integers(0, big, 4 * big), rng.integers(0, big, 4 * big)
+    lo = np.arange(big, n - 1, 2)  # pairs that only an entry of the large tree reaches
+    src = np.concatenate([a, b, lo, lo + 1, rng.integers(0, big, len(lo))])
+    dst = np.concatenate([b, a, lo + 1, lo, lo])
+    order = np.lexsort((rng.random(len(src)), src))
+    ro = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.int32)
+    c = gg.CSR(ro, dst[order].astype(np.int32))
+    whole = sym(n, src, dst)
+    exp = oracle.cc(whole.row_offsets, whole.col_indices)[0]
+    assert len(np.unique(exp)) < n // 100  # nearly one component
+    with gg.Graph(c) as g:
+        np.testing.assert_array_equal(g.cc(hook=True)[0], exp)
+        if n >= 1 << 17:
+            np.testing.assert_array_equal(g.cc()[0], exp)
