@@ -24,6 +24,7 @@
 #include "config.h"
 #include "csc_build.h"
 #include "lbs.h"
+#include "pool.h"
 #include "program_ops.h"
 
 namespace GASengine {
@@ -33,6 +34,24 @@ namespace GASengine {
 inline hipStream_t &engine_stream() {
   static thread_local hipStream_t s = nullptr;
   return s;
+}
+
+// First allocation that failed in a program's Initialize on this thread (which
+// returns nothing): set by program_alloc, returned by the enactor before it
+// launches anything.
+inline hipError_t &program_error() {
+  static thread_local hipError_t e = hipSuccess;
+  return e;
+}
+
+// A program's device array, allocated on first use.  false when there is no
+// memory for it: Initialize then returns without launching anything.
+template <class T>
+inline bool program_alloc(T **p, size_t bytes) {
+  if (*p) return true;
+  const hipError_t e = device_alloc(p, bytes);
+  if (e != hipSuccess && program_error() == hipSuccess) program_error() = e;
+  return e == hipSuccess;
 }
 
 #define GAS_RETURN_IF(expr)            \
@@ -79,22 +98,22 @@ struct Workspace {
     const size_t nn = (size_t)(n > 0 ? n : 1);
     const size_t nw = (size_t)words(n > 0 ? n : 1);
     const size_t np = (nn + kCountTile - 1) / kCountTile + 1;
-    GAS_RETURN_IF(hipMalloc(&frontier[0], nn * 4));
-    GAS_RETURN_IF(hipMalloc(&frontier[1], nn * 4));
-    GAS_RETURN_IF(hipMalloc(&dedup[0], nw * 4));
-    GAS_RETURN_IF(hipMalloc(&dedup[1], nw * 4));
-    GAS_RETURN_IF(hipMalloc(&marks, nw * 32));
-    GAS_RETURN_IF(hipMalloc(&changed, nn));
-    GAS_RETURN_IF(hipMalloc(&gather_tmp, nn * (gather_elem_bytes > 4 ? gather_elem_bytes : 4)));
-    GAS_RETURN_IF(hipMalloc(&scan_local, nn * 4));
-    GAS_RETURN_IF(hipMalloc(&partials, np * 4));
-    GAS_RETURN_IF(hipMalloc(&parts, lbs_partition_entries(n, m) * 4));
-    GAS_RETURN_IF(hipMalloc(&info, sizeof(LbsInfo)));
-    GAS_RETURN_IF(hipMalloc(&sizes, 4 * sizeof(int32_t)));
-    GAS_RETURN_IF(hipMalloc(&counters, 8 * sizeof(unsigned long long)));
+    GAS_RETURN_IF(device_alloc(&frontier[0], nn * 4));
+    GAS_RETURN_IF(device_alloc(&frontier[1], nn * 4));
+    GAS_RETURN_IF(device_alloc(&dedup[0], nw * 4));
+    GAS_RETURN_IF(device_alloc(&dedup[1], nw * 4));
+    GAS_RETURN_IF(device_alloc(&marks, nw * 32));
+    GAS_RETURN_IF(device_alloc(&changed, nn));
+    GAS_RETURN_IF(device_alloc(&gather_tmp, nn * (gather_elem_bytes > 4 ? gather_elem_bytes : 4)));
+    GAS_RETURN_IF(device_alloc(&scan_local, nn * 4));
+    GAS_RETURN_IF(device_alloc(&partials, np * 4));
+    GAS_RETURN_IF(device_alloc(&parts, lbs_partition_entries(n, m) * 4));
+    GAS_RETURN_IF(device_alloc(&info, sizeof(LbsInfo)));
+    GAS_RETURN_IF(device_alloc(&sizes, 4 * sizeof(int32_t)));
+    GAS_RETURN_IF(device_alloc(&counters, 8 * sizeof(unsigned long long)));
     GAS_RETURN_IF(hipHostMalloc(&h_sizes, 8 * sizeof(int32_t)));
-    GAS_RETURN_IF(hipMalloc(&ctl, sizeof(GasCtl)));
-    GAS_RETURN_IF(hipMalloc(&order_words, 2 * kOrderGridMax * sizeof(uint64_t)));
+    GAS_RETURN_IF(device_alloc(&ctl, sizeof(GasCtl)));
+    GAS_RETURN_IF(device_alloc(&order_words, 2 * kOrderGridMax * sizeof(uint64_t)));
     GAS_RETURN_IF(hipHostMalloc(&h_ctl, 2 * sizeof(GasCtl)));
     capacity = n;
     gather_bytes = gather_elem_bytes * nn;
@@ -106,7 +125,7 @@ struct Workspace {
     if (gcarry) (void)hipFree(gcarry);
     gcarry = nullptr;
     gcarry_bytes = 0;
-    GAS_RETURN_IF(hipMalloc(&gcarry, bytes));
+    GAS_RETURN_IF(device_alloc(&gcarry, bytes));
     gcarry_bytes = bytes;
     return hipSuccess;
   }
@@ -118,14 +137,14 @@ struct Workspace {
   }
 
   hipError_t AllocatePreds() {
-    if (!preds) GAS_RETURN_IF(hipMalloc(&preds, (size_t)(capacity > 0 ? capacity : 1) * 4));
+    if (!preds) GAS_RETURN_IF(device_alloc(&preds, (size_t)(capacity > 0 ? capacity : 1) * 4));
     return hipSuccess;
   }
 
   // Misc-value queues handed to Program::Initialize (d_frontier_values[3]).
   hipError_t AllocateValues() {
     for (int i = 0; i < 3; i++)
-      if (!frontier_values[i]) GAS_RETURN_IF(hipMalloc(&frontier_values[i], (size_t)(capacity > 0 ? capacity : 1) * 8));
+      if (!frontier_values[i]) GAS_RETURN_IF(device_alloc(&frontier_values[i], (size_t)(capacity > 0 ? capacity : 1) * 8));
     return hipSuccess;
   }
 
@@ -243,7 +262,7 @@ struct CsrProblem {
     g.edges = edges;
     g.directed = directed;
     auto up = [&](const void *src, size_t bytes, void **dst) -> hipError_t {
-      GAS_RETURN_IF(hipMalloc(dst, bytes > 0 ? bytes : 4));
+      GAS_RETURN_IF(device_alloc(dst, bytes > 0 ? bytes : 4));
       owned.push_back(*dst);
       if (bytes) GAS_RETURN_IF(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
       return hipSuccess;
@@ -261,7 +280,7 @@ struct CsrProblem {
     (void)h_column_offsets;
     if (directed) {
       auto alloc = [&](size_t bytes, void **dst) -> hipError_t {
-        GAS_RETURN_IF(hipMalloc(dst, bytes > 0 ? bytes : 4));
+        GAS_RETURN_IF(device_alloc(dst, bytes > 0 ? bytes : 4));
         owned.push_back(*dst);
         return hipSuccess;
       };

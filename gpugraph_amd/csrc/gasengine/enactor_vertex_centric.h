@@ -276,9 +276,11 @@ class EnactorVertexCentric {
     typename Program::MiscType *vals[3];
     for (int i = 0; i < 3; i++) vals[i] = (typename Program::MiscType *)ws.frontier_values[i];
     engine_stream() = s;
+    program_error() = hipSuccess;
     Program::Initialize(directed, n, (int)g.edges, num_srcs, srcs, (int *)g.row_offsets, (int *)g.column_indices,
                         (int *)g.column_offsets, (int *)g.row_indices, (typename Program::DataType *)g.edge_values,
                         problem.vertex_list, problem.edge_list, keys, vals);
+    GAS_RETURN_IF(program_error());
     GAS_RETURN_IF(hipGetLastError());
     const int32_t nf0 = Program::srcVertex() == SINGLE ? num_srcs : n;
     hipLaunchKernelGGL(k_gas_ctl_init<>, dim3(1), dim3(1), 0, s, ws.ctl, ws.sizes, nf0, threshold,

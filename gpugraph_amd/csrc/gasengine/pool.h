@@ -7,9 +7,10 @@
 // A block may be given back only when nothing on the device can still use it:
 // the caller has synchronised the stream (or the device) that did.  Blocks are
 // kept per device, at most kPoolBlocks of them and kPoolBytes in all (larger
-// ones than kPoolBlock go back to the runtime at once); a failed allocation
-// returns them all to the runtime and tries again.  Any thread may call.
-// Contents are whatever the last user left.
+// ones than kPoolBlock go back to the runtime at once).  Every allocation of
+// the engine and its programs goes through take() or device_alloc(): one that
+// fails for want of memory returns all kept blocks to the runtime and tries
+// again.  Any thread may call.  Contents are whatever the last user left.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -59,7 +60,10 @@ class BlockPool {
       e = hipMalloc(p, want);
     }
     *bytes = e == hipSuccess ? want : 0;
-    if (e != hipSuccess) *p = nullptr;
+    if (e != hipSuccess) {
+      *p = nullptr;
+      (void)hipGetLastError();  // reported by the return value alone
+    }
     return e;
   }
 
@@ -100,6 +104,21 @@ class BlockPool {
   std::vector<Block> blocks_;
   size_t held_ = 0;
 };
+
+// hipMalloc for memory that is freed with hipFree: kept blocks are returned to
+// the runtime before it fails.  *p is null on failure.
+template <class T>
+inline hipError_t device_alloc(T **p, size_t bytes) {
+  void *q = nullptr;
+  hipError_t e = hipMalloc(&q, bytes);
+  if (e == hipErrorOutOfMemory && BlockPool::get().drain()) {
+    (void)hipGetLastError();
+    e = hipMalloc(&q, bytes);
+  }
+  if (e != hipSuccess) (void)hipGetLastError();  // reported by the return value alone
+  *p = e == hipSuccess ? static_cast<T *>(q) : nullptr;
+  return e;
+}
 
 // Scratch of one function that ends with its stream synchronised: released()
 // says so, after which the blocks are kept; otherwise they are freed (which

@@ -39,7 +39,7 @@ struct bfs {
     hipStream_t s = GASengine::engine_stream();
     vertex_list.nodes = nodes;
     vertex_list.edges = edges;
-    if (!vertex_list.d_labels) (void)hipMalloc(&vertex_list.d_labels, sizeof(int) * (size_t)(nodes > 0 ? nodes : 1));
+    if (!GASengine::program_alloc(&vertex_list.d_labels, sizeof(int) * (size_t)(nodes > 0 ? nodes : 1))) return;
     vertex_list.d_labels_src = vertex_list.d_labels;
     (void)GASengine::fill_async<int>(vertex_list.d_labels, INIT_VALUE, nodes, s);
     for (int i = 0; i < num_srcs; i++) (void)GASengine::fill_async<int>(vertex_list.d_labels + srcs[i], 0, 1, s);

@@ -47,8 +47,9 @@ struct cc {
     vertex_list.nodes = nodes;
     vertex_list.edges = edges;
     const size_t nn = (size_t)(nodes > 0 ? nodes : 1);
-    if (!vertex_list.d_dists) (void)hipMalloc(&vertex_list.d_dists, sizeof(DataType) * nn);
-    if (!vertex_list.d_dists_out) (void)hipMalloc(&vertex_list.d_dists_out, sizeof(DataType) * nn);
+    if (!GASengine::program_alloc(&vertex_list.d_dists, sizeof(DataType) * nn) ||
+        !GASengine::program_alloc(&vertex_list.d_dists_out, sizeof(DataType) * nn))
+      return;
     (void)GASengine::sequence_async<int>(vertex_list.d_dists, nodes, s);
     (void)GASengine::sequence_async<int>(vertex_list.d_dists_out, nodes, s);
     (void)GASengine::sequence_async<int>(d_frontier_keys[0], nodes, s);

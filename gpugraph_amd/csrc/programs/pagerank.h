@@ -62,9 +62,10 @@ struct pagerank {
     vertex_list.nodes = nodes;
     vertex_list.edges = edges;
     const size_t nn = (size_t)(nodes > 0 ? nodes : 1);
-    if (!vertex_list.d_dists) (void)hipMalloc(&vertex_list.d_dists, sizeof(DataType) * nn);
-    if (!vertex_list.d_num_out_edge) (void)hipMalloc(&vertex_list.d_num_out_edge, sizeof(int) * nn);
-    if (!vertex_list.d_share) (void)hipMalloc(&vertex_list.d_share, sizeof(DataType) * nn);
+    if (!GASengine::program_alloc(&vertex_list.d_dists, sizeof(DataType) * nn) ||
+        !GASengine::program_alloc(&vertex_list.d_num_out_edge, sizeof(int) * nn) ||
+        !GASengine::program_alloc(&vertex_list.d_share, sizeof(DataType) * nn))
+      return;
     (void)GASengine::fill_async<float>(vertex_list.d_dists, 0.15f, nodes, s);
     (void)GASengine::sequence_async<int>(d_frontier_keys[0], nodes, s);
     if (nodes > 0)

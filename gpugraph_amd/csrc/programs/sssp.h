@@ -45,8 +45,9 @@ struct sssp {
     edge_list.nodes = nodes;
     edge_list.edges = edges;
     const size_t nn = (size_t)(nodes > 0 ? nodes : 1);
-    if (!vertex_list.d_dists) (void)hipMalloc(&vertex_list.d_dists, sizeof(DataType) * nn);
-    if (!vertex_list.d_dists_out) (void)hipMalloc(&vertex_list.d_dists_out, sizeof(DataType) * nn);
+    if (!GASengine::program_alloc(&vertex_list.d_dists, sizeof(DataType) * nn) ||
+        !GASengine::program_alloc(&vertex_list.d_dists_out, sizeof(DataType) * nn))
+      return;
     // The weights stay in the graph's resident value array (the reference
     // copies them into a second device buffer, sssp.h:103-114).
     edge_list.d_weights = d_edge_values;

@@ -46,7 +46,7 @@ struct pagerank_all : pagerank {
                          int *d_frontier_keys[3], MiscType *d_frontier_values[3]) {
     pagerank::Initialize(directed, nodes, edges, num_srcs, srcs, d_row_offsets, d_column_indices, d_column_offsets,
                          d_row_indices, d_edge_values, vertex_list, edge_list, d_frontier_keys, d_frontier_values);
-    if (nodes > 0)
+    if (nodes > 0 && GASengine::program_error() == hipSuccess)
       hipLaunchKernelGGL(pagerank_detail::k_add_in_degree, dim3(GASengine::grid_for(nodes, 256)), dim3(256), 0,
                          GASengine::engine_stream(), d_column_offsets, vertex_list.d_num_out_edge, vertex_list.d_share,
                          nodes);
