@@ -21,7 +21,7 @@ from ._abi import GGError, load_library
 
 __all__ = [
     "CSR", "Graph", "GGError", "load_library", "gen_erdos_renyi", "gen_rmat", "gen_lattice", "read_mtx",
-    "SSSP_INF", "default_options",
+    "SSSP_INF", "default_options", "release_cached_memory",
 ]
 
 SSSP_INF = 100000000  # Algorithms/SSSP/sssp.h:43 INIT_VALUE
@@ -121,6 +121,14 @@ def default_options() -> "_abi.Options":
     o = _abi.Options()
     _abi.check(load_library().gg_default_options(C.byref(o)), "gg_default_options")
     return o
+
+
+def release_cached_memory() -> int:
+    """Return the device memory that the library keeps for the next graph (at
+    most 256 MiB) to the runtime; the number of bytes it was."""
+    n = C.c_int64()
+    _abi.check(load_library().gg_release_cached_memory(C.byref(n)), "gg_release_cached_memory")
+    return n.value
 
 
 def _ptr(a: np.ndarray):

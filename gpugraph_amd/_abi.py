@@ -144,6 +144,7 @@ PROTOTYPES = {
     "gg_version": (C.c_int, []),
     "gg_device_count": (C.c_int, [_I32P]),
     "gg_default_options": (C.c_int, [C.POINTER(Options)]),
+    "gg_release_cached_memory": (C.c_int, [C.POINTER(C.c_int64)]),
     "gg_graph_create": (C.c_int, [C.c_int32, C.c_int64, _P, _P, _P, C.c_int32, C.c_uint32, C.POINTER(_P)]),
     "gg_graph_destroy": (C.c_int, [_P]),
     "gg_graph_set_stream": (C.c_int, [_P, _P]),

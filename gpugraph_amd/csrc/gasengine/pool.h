@@ -1,66 +1,72 @@
 // Device memory kept between uses, for programs that load a graph, query it
 // and drop it again: hipMalloc and hipFree (which waits for the whole device)
 // were more than half of such a pass (a 300k-vertex, 4.8M-edge directed graph
-// loaded, four BFS trees, unloaded: 28 pairs, 3.7 of 6.6 ms; 3.0 ms with
+// loaded, four BFS trees, unloaded: 28 pairs, 3.7 of 6.7 ms; 4.5 ms with
 // the blocks kept).
 //
 // A block may be given back only when nothing on the device can still use it:
 // the caller has synchronised the stream (or the device) that did.  Blocks are
 // kept per device, at most kPoolBlocks of them and kPoolBytes in all (larger
-// ones than kPoolBlock go back to the runtime at once).  Every allocation of
-// the engine and its programs goes through take() or device_alloc(): one that
-// fails for want of memory returns all kept blocks to the runtime and tries
-// again.  Any thread may call.  Contents are whatever the last user left.
+// ones than kPoolBlock go back to the runtime at once, the oldest ones when
+// there is no room).  Every allocation of the engine and its programs goes
+// through take() or device_alloc(): one that fails for want of memory returns
+// all kept blocks to the runtime and tries again.  drain() returns them on
+// request (a program that resets the device does so first: the blocks do not
+// outlive it).  Nothing here allocates host memory or throws.  Any thread may
+// call.  Contents are whatever the last user left.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <mutex>
-#include <vector>
+#include <new>
 
 namespace GASengine {
 
 constexpr size_t kPoolBytes = (size_t)256 << 20;
 constexpr size_t kPoolBlock = (size_t)64 << 20;
-constexpr size_t kPoolBlocks = 128;
+constexpr int kPoolBlocks = 128;
 
 class BlockPool {
  public:
   static BlockPool &get() {
-    static BlockPool *pool = new BlockPool();  // never destroyed: the runtime may be gone by then
+    // Never destroyed (the runtime may be gone by then), no allocation of its own.
+    alignas(BlockPool) static unsigned char storage[sizeof(BlockPool)];
+    static BlockPool *pool = ::new (storage) BlockPool();
     return *pool;
   }
 
   // At least `want` bytes (> 0) on the current device; *bytes gets the size.
   hipError_t take(size_t want, void **p, size_t *bytes) {
+    *p = nullptr;
+    *bytes = 0;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      size_t best = blocks_.size();
-      for (size_t i = 0; i < blocks_.size(); i++) {
+      int best = -1;
+      for (int i = 0; i < count_; i++) {
         const Block &b = blocks_[i];
         if (b.device == dev && b.bytes >= want && b.bytes <= 2 * want &&
-            (best == blocks_.size() || b.bytes < blocks_[best].bytes))
+            (best < 0 || b.bytes < blocks_[best].bytes))
           best = i;
       }
-      if (best < blocks_.size()) {
+      if (best >= 0) {
         *p = blocks_[best].p;
         *bytes = blocks_[best].bytes;
-        held_ -= *bytes;
-        blocks_[best] = blocks_.back();
-        blocks_.pop_back();
+        remove(best);
         return hipSuccess;
       }
     }
     e = hipMalloc(p, want);
-    if (e == hipErrorOutOfMemory && drain()) {
+    if (e == hipErrorOutOfMemory && drain() > 0) {
       (void)hipGetLastError();
       e = hipMalloc(p, want);
     }
-    *bytes = e == hipSuccess ? want : 0;
-    if (e != hipSuccess) {
+    if (e == hipSuccess) {
+      *bytes = want;
+    } else {
       *p = nullptr;
       (void)hipGetLastError();  // reported by the return value alone
     }
@@ -71,27 +77,41 @@ class BlockPool {
   void give(void *p, size_t bytes) {
     if (!p) return;
     int dev = 0;
-    if (bytes <= kPoolBlock && hipGetDevice(&dev) == hipSuccess) {
-      std::lock_guard<std::mutex> lock(mutex_);
-      if (held_ + bytes <= kPoolBytes && blocks_.size() < kPoolBlocks) {
-        blocks_.push_back({p, bytes, dev});
-        held_ += bytes;
-        return;
-      }
+    if (bytes > kPoolBlock || hipGetDevice(&dev) != hipSuccess) {
+      (void)hipFree(p);
+      return;
     }
-    (void)hipFree(p);
-  }
-
-  // Frees every kept block; whether there was one.
-  bool drain() {
-    std::vector<Block> old;
+    void *old[kPoolBlocks];
+    int olds = 0;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      old.swap(blocks_);
+      while (count_ == kPoolBlocks || held_ + bytes > kPoolBytes) {
+        old[olds++] = blocks_[0].p;
+        remove(0);
+      }
+      blocks_[count_++] = {p, bytes, dev};
+      held_ += bytes;
+    }
+    for (int i = 0; i < olds; i++) (void)hipFree(old[i]);
+  }
+
+  // Frees every kept block; the bytes they held.
+  size_t drain() {
+    void *old[kPoolBlocks];
+    int olds = 0;
+    size_t bytes = 0;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      while (olds < count_) {
+        old[olds] = blocks_[olds].p;
+        olds++;
+      }
+      bytes = held_;
+      count_ = 0;
       held_ = 0;
     }
-    for (const Block &b : old) (void)hipFree(b.p);
-    return !old.empty();
+    for (int i = 0; i < olds; i++) (void)hipFree(old[i]);
+    return bytes;
   }
 
  private:
@@ -100,8 +120,14 @@ class BlockPool {
     size_t bytes;
     int device;
   };
+  void remove(int at) {  // the order of age is kept
+    held_ -= blocks_[at].bytes;
+    count_--;
+    for (int i = at; i < count_; i++) blocks_[i] = blocks_[i + 1];
+  }
   std::mutex mutex_;
-  std::vector<Block> blocks_;
+  Block blocks_[kPoolBlocks];  // oldest first
+  int count_ = 0;
   size_t held_ = 0;
 };
 
@@ -111,7 +137,7 @@ template <class T>
 inline hipError_t device_alloc(T **p, size_t bytes) {
   void *q = nullptr;
   hipError_t e = hipMalloc(&q, bytes);
-  if (e == hipErrorOutOfMemory && BlockPool::get().drain()) {
+  if (e == hipErrorOutOfMemory && BlockPool::get().drain() > 0) {
     (void)hipGetLastError();
     e = hipMalloc(&q, bytes);
   }
@@ -125,30 +151,39 @@ inline hipError_t device_alloc(T **p, size_t bytes) {
 // waits for the device).
 class PoolScratch {
  public:
+  PoolScratch() = default;
+  PoolScratch(const PoolScratch &) = delete;
+  PoolScratch &operator=(const PoolScratch &) = delete;
   ~PoolScratch() {
-    for (const auto &b : blocks_) {
+    for (int i = 0; i < count_; i++) {
       if (idle_)
-        BlockPool::get().give(b.p, b.bytes);
+        BlockPool::get().give(blocks_[i].p, blocks_[i].bytes);
       else
-        (void)hipFree(b.p);
+        (void)hipFree(blocks_[i].p);
     }
   }
+  // At most kMax blocks.
   template <class T>
   hipError_t alloc(T **p, size_t bytes) {
+    *p = nullptr;
+    if (count_ == kMax) return hipErrorInvalidValue;
     Block b{nullptr, 0};
     const hipError_t e = BlockPool::get().take(bytes ? bytes : 4, &b.p, &b.bytes);
+    if (e != hipSuccess) return e;
     *p = static_cast<T *>(b.p);
-    if (e == hipSuccess) blocks_.push_back(b);
-    return e;
+    blocks_[count_++] = b;
+    return hipSuccess;
   }
   void released() { idle_ = true; }
 
  private:
+  static constexpr int kMax = 8;
   struct Block {
     void *p;
     size_t bytes;
   };
-  std::vector<Block> blocks_;
+  Block blocks_[kMax];
+  int count_ = 0;
   bool idle_ = false;
 };
 

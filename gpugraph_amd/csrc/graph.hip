@@ -466,6 +466,13 @@ int gg_default_options(gg_options *o) {
   return GG_OK;
 }
 
+int gg_release_cached_memory(int64_t *bytes) {
+  gg::clear_error();
+  const size_t held = GASengine::BlockPool::get().drain();
+  if (bytes) *bytes = (int64_t)held;
+  return GG_OK;
+}
+
 int gg_graph_create(int32_t n, int64_t m, const int32_t *row_offsets, const int32_t *col_indices, const void *values,
                     int32_t value_dtype, uint32_t flags, gg_graph **out) {
   gg::clear_error();

@@ -114,6 +114,12 @@ const char *gg_last_error(void);
 int gg_version(void);                     /* major*10000 + minor*100 + patch */
 int gg_device_count(int32_t *count);
 int gg_default_options(gg_options *out);
+/* The library keeps device memory of destroyed graphs and of scratch for the
+ * next graph (at most 256 MiB, in blocks of at most 64 MiB) and returns it to
+ * the runtime when an allocation of its own fails.  This returns it now, for
+ * other users of the device, and before a hipDeviceReset.  *bytes (may be
+ * NULL): how much it was. */
+int gg_release_cached_memory(int64_t *bytes);
 
 /* ---- graph -------------------------------------------------------------- */
 /* Replaces CsrProblem::FromHostProblem (GASengine/csr_problem.cuh:512-839):

@@ -21,3 +21,16 @@ def test_engine_and_programs_report_failed_allocations(tmp_path):
     assert r.returncode == 0, r.stderr[-3000:]
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout[-3000:] + r.stderr[-1000:]
+
+
+def test_block_pool(tmp_path):
+    """Reuse, bounds, eviction of the oldest, return on demand and when memory
+    is short, several threads, on a host-side device of limited memory."""
+    exe = tmp_path / "check"
+    native = os.path.join(ROOT, "tests", "native")
+    r = subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-I", os.path.join(native, "fake_hip"), "-I",
+                        os.path.join(ROOT, "gpugraph_amd", "csrc"), os.path.join(native, "pool_check.cpp"), "-o", str(exe),
+                        "-lpthread"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-3000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout[-3000:]

@@ -48,3 +48,21 @@ def test_handles_in_turn(gpu_available, threads):
     for t in ts:
         t.join()
     assert not errors, errors
+
+
+def test_release_cached_memory(gpu_available):
+    """Memory of a dropped handle is kept and comes back on request."""
+    import torch
+
+    c = gg.gen_rmat(16, 16, undirected=True, seed=95)
+    gg.release_cached_memory()
+    with gg.Graph(c) as g:
+        exp = g.bfs(1)[0]
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    held = gg.release_cached_memory()
+    assert 4 * c.m < held <= 256 << 20
+    assert torch.cuda.mem_get_info()[0] > before
+    assert gg.release_cached_memory() == 0
+    with gg.Graph(c) as g:
+        np.testing.assert_array_equal(g.bfs(1)[0], exp)
