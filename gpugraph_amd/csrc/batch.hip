@@ -330,21 +330,24 @@ __global__ void k_bs_clear(BatchState *st) {
 }
 
 __global__ void k_bs_swap(BatchState *st, const LbsInfo *info, int32_t max_iter) {
+  int32_t *const q_cur = st->q_cur, *const q_nxt = st->q_nxt;
+  uint32_t *const ub_cur = st->ub_cur, *const ub_nxt = st->ub_nxt;
+  uint32_t *const act_cur = st->act_cur, *const act_nxt = st->act_nxt;
+  const int32_t next = st->nxt_size, iters = st->sssp_iters + 1;
+  const unsigned long long edges = st->edges + (unsigned long long)info->edges;
   if (st->sssp_done) return;
-  st->edges += (unsigned long long)info->edges;
-  int32_t *q = st->q_cur;
-  st->q_cur = st->q_nxt;
-  st->q_nxt = q;
-  uint32_t *b = st->ub_cur;
-  st->ub_cur = st->ub_nxt;
-  st->ub_nxt = b;
-  uint32_t *a = st->act_cur;
-  st->act_cur = st->act_nxt;
-  st->act_nxt = a;
-  st->cur_size = st->nxt_size;
+  scalar_loads_done();
+  st->edges = edges;
+  st->q_cur = q_nxt;
+  st->q_nxt = q_cur;
+  st->ub_cur = ub_nxt;
+  st->ub_nxt = ub_cur;
+  st->act_cur = act_nxt;
+  st->act_nxt = act_cur;
+  st->cur_size = next;
   st->nxt_size = 0;
-  st->sssp_iters++;
-  if (st->cur_size == 0 || st->sssp_iters >= max_iter) st->sssp_done = 1;
+  st->sssp_iters = iters;
+  if (next == 0 || iters >= max_iter) st->sssp_done = 1;
 }
 
 // Vertex-major rows -> instance-major output: in[row(v)][KW] -> out[i][v] for
@@ -584,7 +587,10 @@ k_ppr_long_finish(PprArgs a, BatchState *st, const int32_t *__restrict__ longv, 
 // 64 threads: close the iteration for every instance.
 __global__ void k_ppr_finalize(BatchState *st, int32_t nseeds, double tol, int32_t max_iter) {
   __shared__ double s_max[kPprMax];
+  float *const r_cur = st->r_cur, *const r_nxt = st->r_nxt;
+  const int32_t iters = st->ppr_iters + 1;
   if (st->ppr_done) return;
+  scalar_loads_done();
   const int l = threadIdx.x;
   double r = 0.0, dg = 0.0;
   for (int q = 0; q < kStripes; q++) {
@@ -601,11 +607,10 @@ __global__ void k_ppr_finalize(BatchState *st, int32_t nseeds, double tol, int32
     double mx = 0.0;
     for (int j = 0; j < kPprMax; j++) mx = fmax(mx, s_max[j]);
     st->resid_last_max = mx;
-    float *t = st->r_cur;
-    st->r_cur = st->r_nxt;
-    st->r_nxt = t;
-    st->ppr_iters++;
-    if (mx <= tol || st->ppr_iters >= max_iter) st->ppr_done = 1;
+    st->r_cur = r_nxt;
+    st->r_nxt = r_cur;
+    st->ppr_iters = iters;
+    if (mx <= tol || iters >= max_iter) st->ppr_done = 1;
   }
 }
 

@@ -54,7 +54,7 @@ constexpr int kBlock = 256;
 constexpr int kPullDiv = 8;  // pull while the frontier exceeds n / kPullDiv
 constexpr int kCcStride = 16;  // 128 bytes between the stripes of a counter
 
-struct CcState {
+struct CcLoop {
   int32_t *q_cur, *q_nxt;
   uint32_t *b_cur, *b_nxt;  // dedup bitmaps of q_cur / q_nxt
   int32_t cur_size, nxt_size;
@@ -65,9 +65,11 @@ struct CcState {
   int32_t pull, pulls;                // this iteration pulls; pull iterations so far
   int32_t prev_pull, pull_skip;       // last iteration pulled; pull kernel off (done || !pull)
   int32_t fill;                       // queue fill position of the bitmap compaction
-  unsigned long long pull_changed;    // vertices changed by this iteration's pull
+};
+struct CcState : CcLoop {
   // Striped per-workgroup sums (GASengine::block_counter_add, stride
-  // kCcStride), folded into edges / pull_changed by k_lp_swap.
+  // kCcStride) of an iteration, folded by k_lp_swap: edges, and the vertices a
+  // pull changed.
   unsigned long long edge_stripes[kStripes * kCcStride];
   unsigned long long changed_stripes[kStripes * kCcStride];
 };
@@ -89,7 +91,6 @@ __global__ void k_lp_state_init(CcState *st, int32_t *q0, int32_t *q1, uint32_t 
   st->prev_pull = 0;
   st->pull_skip = !st->pull || st->done;
   st->fill = 0;
-  st->pull_changed = 0;
   for (int q = 0; q < kStripes * kCcStride; q++) st->edge_stripes[q] = st->changed_stripes[q] = 0;
 }
 
@@ -175,7 +176,7 @@ k_lp_expand(CcState *st, const int32_t *__restrict__ ro, const int32_t *__restri
 struct CcPullOp {
   const int32_t *nbr;
   int32_t *label;
-  CcState *st;                    // output bitmap st->b_nxt (cleared before the pull), count st->pull_changed
+  CcState *st;                    // output bitmap st->b_nxt (cleared before the pull), count st->changed_stripes
   unsigned long long count;
 
   struct Edge {
@@ -252,40 +253,35 @@ k_lp_prep(CcState *st, int32_t words) {
   }
 }
 
-__global__ void k_lp_swap(CcState *st, int32_t n, int64_t m, int32_t max_iter) {
-  if (st->done) return;
-  unsigned long long pushed = 0, changed = 0;
-  for (int q = 0; q < kStripes; q++) {
-    pushed += st->edge_stripes[q * kCcStride];
-    changed += st->changed_stripes[q * kCcStride];
-    st->edge_stripes[q * kCcStride] = 0;
-    st->changed_stripes[q * kCcStride] = 0;
-  }
-  st->edges += pushed;
-  st->pull_changed += changed;
-  if (st->pull) {
-    st->edges += (unsigned long long)m;
-    st->pulls++;
-    st->nxt_size = (int32_t)st->pull_changed;
-    st->pull_changed = 0;
-  } else {
-    st->push_frontier += (unsigned long long)st->cur_size;
-  }
-  st->prev_pull = st->pull;
+// End of an iteration (one wave): folds the sums, swaps the buffers, picks the
+// next direction.
+__global__ void __launch_bounds__(kWave) k_lp_swap(CcState *st, int32_t n, int64_t m, int32_t max_iter) {
+  const CcLoop old = *st;
+  if (old.done) return;
+  const unsigned long long pushed = take_stripes<kCcStride>(st->edge_stripes);
+  const unsigned long long changed = take_stripes<kCcStride>(st->changed_stripes);
+  scalar_loads_done();
+  if (threadIdx.x != 0) return;
+  const int32_t next = old.pull ? (int32_t)changed : old.nxt_size;
+  const int32_t pull = next > n / kPullDiv, done = next == 0 || old.iters + 1 >= max_iter;
+  st->edges = old.edges + pushed + (old.pull ? (unsigned long long)m : 0ull);
+  if (old.pull)
+    st->pulls = old.pulls + 1;
+  else
+    st->push_frontier = old.push_frontier + (unsigned long long)old.cur_size;
+  st->prev_pull = old.pull;
   st->fill = 0;
-  int32_t *q = st->q_cur;
-  st->q_cur = st->q_nxt;
-  st->q_nxt = q;
-  uint32_t *b = st->b_cur;
-  st->b_cur = st->b_nxt;
-  st->b_nxt = b;
-  st->frontier_total += (unsigned long long)st->cur_size;
-  st->cur_size = st->nxt_size;
+  st->q_cur = old.q_nxt;
+  st->q_nxt = old.q_cur;
+  st->b_cur = old.b_nxt;
+  st->b_nxt = old.b_cur;
+  st->frontier_total = old.frontier_total + (unsigned long long)old.cur_size;
+  st->cur_size = next;
   st->nxt_size = 0;
-  st->iters++;
-  st->pull = st->cur_size > n / kPullDiv;
-  if (st->cur_size == 0 || st->iters >= max_iter) st->done = 1;
-  st->pull_skip = !st->pull || st->done;
+  st->iters = old.iters + 1;
+  st->pull = pull;
+  st->done = done;
+  st->pull_skip = !pull || done;
 }
 
 }  // namespace
@@ -351,7 +347,7 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
                          label, g->opt.wave_degree);
       hipLaunchKernelGGL((k_pull_staged<CcPullOp, int32_t>), dim3(grid), dim3(kExpandBlock), 0, s, pull_op,
                          g->dg.row_offsets, n, g->m, parts, &st->pull_skip);
-      hipLaunchKernelGGL(k_lp_swap, dim3(1), dim3(1), 0, s, st, n, g->m, max_iter);
+      hipLaunchKernelGGL(k_lp_swap, dim3(1), dim3(kWave), 0, s, st, n, g->m, max_iter);
     }
     const hipError_t cap = hipStreamEndCapture(s, &graph);
     hipError_t inst = hipErrorUnknown;

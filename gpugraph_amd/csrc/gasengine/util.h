@@ -166,6 +166,30 @@ template <int STRIDE = kCounterSlots, class T>
 __device__ __forceinline__ T *stripe_of(T *counter) {
   return counter + (int)(blockIdx.x % kStripes) * STRIDE;
 }
+// Fold a striped sum and clear its stripes (one wave, a lane a stripe; every
+// lane gets the sum).  A single thread doing this is slower (16 loads one by
+// one) and depends on scalar_loads_done.
+template <int STRIDE = kCounterSlots, class T>
+__device__ __forceinline__ T take_stripes(T *counter) {
+  static_assert(kStripes <= kWave, "a lane per stripe");
+  const int q = lane_id();
+  T t = 0;
+  if (q < kStripes) {
+    t = counter[q * STRIDE];
+    counter[q * STRIDE] = 0;
+  }
+#pragma unroll
+  for (int off = kStripes / 2; off > 0; off >>= 1) t += __shfl_xor(t, off);
+  return __shfl(t, 0);
+}
+
+// Waits for the scalar loads issued so far.  A word of uniform address may be
+// read through the scalar cache, which is not ordered with vector stores, and
+// the compiler does not wait before it stores to the same word: kernels that
+// replace state they have read (the controllers, one thread or one wave) read
+// all of it, call this, and store.
+__device__ __forceinline__ void scalar_loads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 template <int STRIDE = kCounterSlots, class T>
 __device__ __forceinline__ T stripe_sum(const T *counter) {
   T t = counter[0];

@@ -67,28 +67,6 @@ struct PrState {
   double sq_acc[kStripes * kPrStride];
 };
 
-// Fold a striped FP64 sum and clear its stripes (one wave, a lane a stripe;
-// every lane gets the sum).  A single thread doing this is slower (16 loads
-// one by one) and not safe: its loads have a uniform address, so they may go
-// through the scalar cache, which is not ordered with the vector stores that
-// clear the same words.
-__device__ __forceinline__ double take_stripes(double *acc) {
-  static_assert(kStripes <= kWave, "a lane per stripe");
-  const int q = lane_id();
-  double t = 0.0;
-  if (q < kStripes) {
-    t = acc[q * kPrStride];
-    acc[q * kPrStride] = 0.0;
-  }
-#pragma unroll
-  for (int off = kStripes / 2; off > 0; off >>= 1) t += __shfl_xor(t, off);
-  return __shfl(t, 0);
-}
-
-// Waits for the scalar loads issued so far: a state word read through the
-// scalar cache must have arrived before a vector store replaces it.
-__device__ __forceinline__ void scalar_loads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 template <int BLOCK>
 __device__ __forceinline__ void block_add_f64(double *p, double v) {
   __shared__ double red[BLOCK / kWave];
@@ -257,7 +235,7 @@ __global__ void __launch_bounds__(kWave) k_pr_finalize(PrState *st, double tol, 
   if (st->done) return;
   const double limit = tol * st->scale;
   const int32_t iters = st->iters + 1;
-  const double resid = take_stripes(st->resid_acc), aux = take_stripes(st->aux_acc);
+  const double resid = take_stripes<kPrStride>(st->resid_acc), aux = take_stripes<kPrStride>(st->aux_acc);
   scalar_loads_done();
   if (threadIdx.x != 0) return;
   st->resid_last = resid;
@@ -296,7 +274,7 @@ k_adj_finalize(PrState *st, double tol, int32_t max_iter, int32_t n, double d) {
   const double gap = d * st->gap;                           // lambda' minus the plain iterate
   const int32_t iters = st->iters + 1;
   bool plain_only = st->plain_only != 0;
-  const double plain = take_stripes(st->resid_acc), sq = take_stripes(st->sq_acc), sum = take_stripes(st->aux_acc);
+  const double plain = take_stripes<kPrStride>(st->resid_acc), sq = take_stripes<kPrStride>(st->sq_acc), sum = take_stripes<kPrStride>(st->aux_acc);
   scalar_loads_done();
   if (threadIdx.x != 0) return;
   const double bound = sqrt((double)n * sq), rsum = sum - read;
@@ -351,7 +329,7 @@ k_pr_init(float *r0, float *x0, const float *tele, const float *inv_out, int32_t
 }
 
 __global__ void __launch_bounds__(kWave) k_pr_start(PrState *st, int adjoint) {
-  const double scale = take_stripes(st->scale_acc), aux = take_stripes(st->aux_acc);
+  const double scale = take_stripes<kPrStride>(st->scale_acc), aux = take_stripes<kPrStride>(st->aux_acc);
   if (threadIdx.x != 0) return;
   st->scale = !adjoint || scale == 0.0 ? 1.0 : scale;
   st->aux_cur = aux;
