@@ -50,7 +50,7 @@ static constexpr bool kWithValue = false;
 static constexpr bool kMarkPredecessors = false;
 #elif defined(GG_PROGRAM_PAGERANK)
 #include "programs/pagerank.h"
-typedef pagerank Program;
+typedef pagerank_share Program;
 static const char *kProgram = "PageRank";
 static constexpr bool kWithValue = false;
 static constexpr bool kMarkPredecessors = false;

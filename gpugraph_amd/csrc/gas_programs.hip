@@ -54,7 +54,7 @@ struct Slot<cc> {
   static constexpr int default_threshold = 10000;  // Algorithms/CC/register.h:39
 };
 template <>
-struct Slot<pagerank> {
+struct Slot<pagerank_share> {
   static constexpr int index = 3;
   static constexpr const char *name = "pagerank_ref";
   static constexpr int default_threshold = 1000;  // Algorithms/PageRank/register.h:40
@@ -73,7 +73,7 @@ struct Slot<cc_weak> {
   static constexpr int default_threshold = 10000;
 };
 template <>
-struct Slot<pagerank_all> {
+struct Slot<pagerank_all_share> {
   static constexpr int index = 6;
   static constexpr const char *name = "pagerank_all";
   static constexpr int default_threshold = 1000;
@@ -371,8 +371,8 @@ int gg_pagerank_reference(gg_graph *g, float *rank, uint32_t flags, gg_stats *st
   const bool all = flags & GG_PR_ALL_EDGES;
   GG_CHECK_ARG(!all || g->directed, "GG_PR_ALL_EDGES is for directed graphs");
   auto run = [&](float *o, uint32_t f) {
-    return all ? run_program<pagerank_all>(g, 0, nullptr, o, f, stats, 0.0f, false)
-               : run_program<pagerank>(g, 0, nullptr, o, f, stats, 0.0f, false);
+    return all ? run_program<pagerank_all_share>(g, 0, nullptr, o, f, stats, 0.0f, false)
+               : run_program<pagerank_share>(g, 0, nullptr, o, f, stats, 0.0f, false);
   };
   if (!g->reordered) return run(rank, flags);
   return with_mapped_output(g, rank, flags,

@@ -13,13 +13,13 @@
 #include "../gasengine/csr_problem.h"
 
 namespace pagerank_detail {
-static __global__ void k_out_degree(const int *__restrict__ ro, int *__restrict__ deg, float *__restrict__ share,
-                                    int n) {
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-    const int d = ro[v + 1] - ro[v];
-    deg[v] = d;
-    share[v] = 0.15f / (float)d;
-  }
+static __global__ void k_out_degree(const int *__restrict__ ro, int *__restrict__ deg, int n) {
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) deg[v] = ro[v + 1] - ro[v];
+}
+static __global__ void k_shares(const float *__restrict__ rank, const int *__restrict__ deg, float *__restrict__ share,
+                                int n) {
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
+    share[v] = rank[v] / (float)deg[v];
 }
 }  // namespace pagerank_detail
 
@@ -38,12 +38,7 @@ struct pagerank {
     int edges;
     DataType *d_dists;
     int *d_num_out_edge;
-    // rank / degree, divided once when the rank is set: what a gather edge
-    // reads.  The gather is bound by its random 4-byte reads (about 250 G/s
-    // out of the L2s), two per edge with rank and degree read apart: 97 ->
-    // 58 us per gather over 12M edges.
-    DataType *d_share;
-    VertexType() : nodes(0), edges(0), d_dists(nullptr), d_num_out_edge(nullptr), d_share(nullptr) {}
+    VertexType() : nodes(0), edges(0), d_dists(nullptr), d_num_out_edge(nullptr) {}
   };
 
   struct EdgeType {
@@ -63,24 +58,23 @@ struct pagerank {
     vertex_list.edges = edges;
     const size_t nn = (size_t)(nodes > 0 ? nodes : 1);
     if (!GASengine::program_alloc(&vertex_list.d_dists, sizeof(DataType) * nn) ||
-        !GASengine::program_alloc(&vertex_list.d_num_out_edge, sizeof(int) * nn) ||
-        !GASengine::program_alloc(&vertex_list.d_share, sizeof(DataType) * nn))
+        !GASengine::program_alloc(&vertex_list.d_num_out_edge, sizeof(int) * nn))
       return;
     (void)GASengine::fill_async<float>(vertex_list.d_dists, 0.15f, nodes, s);
     (void)GASengine::sequence_async<int>(d_frontier_keys[0], nodes, s);
     if (nodes > 0)
       hipLaunchKernelGGL(pagerank_detail::k_out_degree, dim3(GASengine::grid_for(nodes, 256)), dim3(256), 0, s,
-                         d_row_offsets, vertex_list.d_num_out_edge, vertex_list.d_share, nodes);
+                         d_row_offsets, vertex_list.d_num_out_edge, nodes);
   }
 
   static void Release(VertexType &vertex_list, EdgeType &) {
     if (vertex_list.d_dists) (void)hipFree(vertex_list.d_dists);
     if (vertex_list.d_num_out_edge) (void)hipFree(vertex_list.d_num_out_edge);
-    if (vertex_list.d_share) (void)hipFree(vertex_list.d_share);
     vertex_list.d_dists = nullptr;
     vertex_list.d_num_out_edge = nullptr;
-    vertex_list.d_share = nullptr;
   }
+
+  static void DegreesSet(VertexType &) {}
 
   static SrcVertex srcVertex() { return ALL; }
   static GatherEdges gatherOverEdges() { return GATHER_IN_EDGES; }
@@ -91,7 +85,8 @@ struct pagerank {
   struct gather_edge {
     __device__ void operator()(const int, const int, const int neighbor_id_in, VertexType &vertex_list, EdgeType &,
                                GatherType &new_value) {
-      new_value = vertex_list.d_share[neighbor_id_in];
+      DataType nb_dist = vertex_list.d_dists[neighbor_id_in];
+      new_value = nb_dist / (DataType)vertex_list.d_num_out_edge[neighbor_id_in];
     }
   };
 
@@ -106,7 +101,6 @@ struct pagerank {
       const DataType newvalue = 0.15f + (1.0f - 0.15f) * gathervalue;
       changed = fabsf(oldvalue - newvalue) < 0.01f ? 0 : 1;
       vertex_list.d_dists[vertex_id] = newvalue;
-      vertex_list.d_share[vertex_id] = newvalue / (DataType)vertex_list.d_num_out_edge[vertex_id];
     }
   };
 
@@ -135,4 +129,57 @@ struct pagerank {
   }
 
   static DataType *resultPointer(VertexType &vertex_list) { return vertex_list.d_dists; }
+};
+
+// The same program with rank / degree kept beside the rank, divided once when
+// the rank is set: one word per gather edge.  The gather is bound by its random
+// 4-byte reads (about 250 G/s out of the L2s), two per edge with rank and
+// degree read apart: 97 -> 58 us per gather over 12M edges.  What the library
+// and the driver run.  A program that derives from pagerank and sets ranks or
+// degrees itself needs nothing of this; one that derives from here keeps
+// d_share up to date.
+struct pagerank_share : pagerank {
+  struct VertexType : pagerank::VertexType {
+    DataType *d_share = nullptr;
+  };
+
+  static void Initialize(const int directed, const int nodes, const int edges, int num_srcs, int *srcs,
+                         int *d_row_offsets, int *d_column_indices, int *d_column_offsets, int *d_row_indices,
+                         DataType *d_edge_values, VertexType &vertex_list, EdgeType &edge_list,
+                         int *d_frontier_keys[3], MiscType *d_frontier_values[3]) {
+    if (!GASengine::program_alloc(&vertex_list.d_share, sizeof(DataType) * (size_t)(nodes > 0 ? nodes : 1))) return;
+    pagerank::Initialize(directed, nodes, edges, num_srcs, srcs, d_row_offsets, d_column_indices, d_column_offsets,
+                         d_row_indices, d_edge_values, vertex_list, edge_list, d_frontier_keys, d_frontier_values);
+    if (GASengine::program_error() == hipSuccess) DegreesSet(vertex_list);
+  }
+
+  // After a change of the degrees (or the ranks) outside apply.
+  static void DegreesSet(VertexType &vertex_list) {
+    if (vertex_list.nodes > 0)
+      hipLaunchKernelGGL(pagerank_detail::k_shares, dim3(GASengine::grid_for(vertex_list.nodes, 256)), dim3(256), 0,
+                         GASengine::engine_stream(), vertex_list.d_dists, vertex_list.d_num_out_edge,
+                         vertex_list.d_share, vertex_list.nodes);
+  }
+
+  static void Release(VertexType &vertex_list, EdgeType &edge_list) {
+    pagerank::Release(vertex_list, edge_list);
+    if (vertex_list.d_share) (void)hipFree(vertex_list.d_share);
+    vertex_list.d_share = nullptr;
+  }
+
+  struct gather_edge {
+    __device__ void operator()(const int, const int, const int neighbor_id_in, VertexType &vertex_list, EdgeType &,
+                               GatherType &new_value) {
+      new_value = vertex_list.d_share[neighbor_id_in];
+    }
+  };
+
+  struct apply {
+    __device__ void operator()(const int vertex_id, const int iteration, GatherType gathervalue,
+                               VertexType &vertex_list, EdgeType &edge_list, char &changed) {
+      pagerank::apply()(vertex_id, iteration, gathervalue, vertex_list, edge_list, changed);
+      vertex_list.d_share[vertex_id] =
+          vertex_list.d_dists[vertex_id] / (DataType)vertex_list.d_num_out_edge[vertex_id];
+    }
+  };
 };

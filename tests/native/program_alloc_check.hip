@@ -160,6 +160,8 @@ int main() {
   program<bfs_reverse>("bfs_reverse");
   program<cc_weak>("cc_weak");
   program<pagerank_all>("pagerank_all");
+  program<pagerank_share>("pagerank_share");
+  program<pagerank_all_share>("pagerank_all_share");
   // A block kept by the pool is what is missing: it is returned, and the
   // allocation succeeds.
   void *p = nullptr;
