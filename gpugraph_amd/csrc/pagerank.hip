@@ -257,24 +257,35 @@ __global__ void __launch_bounds__(kWave) k_pr_finalize(PrState *st, double tol, 
 //    takes more sweeps than the plain iteration.  The result is then its
 //    iterate, lambda' - d gap (offset).
 // At max_iter the plain iterate and its residual are returned as well.
-// From sweep kShiftTrial on, a residual whose bound is not below the plain
-// iteration's own says that the rest converges no faster than the constant
-// part (|lambda_2| = 1: cycles, stars, several closed components); the run
-// then goes back to the plain iterate (sigma = -gap) and stays with it, since
-// a shifted vector keeps changing in its last bits where a plain one settles
-// (star of 1500 vertices: 90 sweeps with the shift to the end, 78 plain).
-// No shift once the residual's sum is at the rounding level of the FP32
-// vectors (2^-24 ||c||_1): both tests then see a settled iteration.
+// A run that neither test has ended goes back to the plain iterate (sigma =
+// -gap) and on from there by plain sweeps (gap 0), to stop where a plain run
+// stops, in two cases: from sweep kShiftTrial on, when the residual's bound is
+// not below the plain iteration's own (the rest converges no faster than the
+// constant part: |lambda_2| = 1 as in cycles, stars, several closed components),
+// and at sweep shift_last(d), where plain sweeps have left 1e-5 of their error.
+// By then the residual is down to the rounding of the FP32 vectors, which a
+// shift keeps changing in their last bits where plain sweeps settle, while the
+// plain iterate's own steps are still tens of roundings large.  (Forest of 100k
+// vertices, d = 0.95, tol 2e-7, c = 1: no end with the shift kept on, 268 sweeps
+// so and plain.)  A tolerance below kSettled asks for vectors that no longer
+// change: such a run is plain from its first sweep.
+// No shift either while the residual's sum is at the rounding level.
 constexpr int kShiftTrial = 16;
+inline int32_t shift_last(double d) {
+  return d > 0.01 ? std::max(2, (int32_t)std::ceil(std::log(1e-5) / std::log(d))) : 2;
+}
+constexpr double kFp32Rounding = 0x1p-24;
+constexpr double kSettled = 0x1p-32;
 __global__ void __launch_bounds__(kWave)
-k_adj_finalize(PrState *st, double tol, int32_t max_iter, int32_t n, double d) {
+k_adj_finalize(PrState *st, double tol, int32_t max_iter, int32_t n, double d, int32_t last) {
   if (st->done) return;
-  const double limit = tol * st->scale, noise = 0x1p-24 * st->scale;
+  const double limit = tol * st->scale, noise = kFp32Rounding * st->scale;
   const double read = st->aux_cur + (double)n * st->shift;  // sum of the vector this sweep read
   const double gap = d * st->gap;                           // lambda' minus the plain iterate
   const int32_t iters = st->iters + 1;
   bool plain_only = st->plain_only != 0;
-  const double plain = take_stripes<kPrStride>(st->resid_acc), sq = take_stripes<kPrStride>(st->sq_acc), sum = take_stripes<kPrStride>(st->aux_acc);
+  const double plain = take_stripes<kPrStride>(st->resid_acc), sq = take_stripes<kPrStride>(st->sq_acc);
+  const double sum = take_stripes<kPrStride>(st->aux_acc);
   scalar_loads_done();
   if (threadIdx.x != 0) return;
   const double bound = sqrt((double)n * sq), rsum = sum - read;
@@ -287,17 +298,21 @@ k_adj_finalize(PrState *st, double tol, int32_t max_iter, int32_t n, double d) {
     st->done = 1;
     return;
   }
-  if (iters >= kShiftTrial && bound >= plain) plain_only = true;
-  double shift = 0.0;
-  if (plain_only)
-    shift = -gap;
-  else if (isfinite(rsum) && fabs(rsum) > noise)
-    shift = d / (1.0 - d) * rsum / (double)n;
-  shift = (double)(float)shift;
+  double shift = 0.0, next_gap = gap;
+  if (!plain_only) {
+    if (iters >= last || (iters >= kShiftTrial && bound >= plain)) {
+      plain_only = true;
+      shift = (double)(float)-gap;
+      next_gap = 0.0;
+    } else {
+      if (isfinite(rsum) && fabs(rsum) > noise) shift = (double)(float)(d / (1.0 - d) * rsum / (double)n);
+      next_gap = gap + shift;
+    }
+  }
   st->resid_last = plain;
   st->plain_only = plain_only;
   st->shift = shift;
-  st->gap = gap + shift;
+  st->gap = next_gap;
 }
 
 __global__ void k_add_offset(float *__restrict__ x, const PrState *__restrict__ st, int32_t n) {
@@ -328,13 +343,13 @@ k_pr_init(float *r0, float *x0, const float *tele, const float *inv_out, int32_t
   block_add_f64<kRowBlock>(st->scale_acc, mag);
 }
 
-__global__ void __launch_bounds__(kWave) k_pr_start(PrState *st, int adjoint) {
+__global__ void __launch_bounds__(kWave) k_pr_start(PrState *st, int adjoint, int plain_only) {
   const double scale = take_stripes<kPrStride>(st->scale_acc), aux = take_stripes<kPrStride>(st->aux_acc);
   if (threadIdx.x != 0) return;
   st->scale = !adjoint || scale == 0.0 ? 1.0 : scale;
   st->aux_cur = aux;
   st->offset = st->shift = st->gap = 0.0;
-  st->plain_only = 0;
+  st->plain_only = plain_only;
   st->resid_last = INFINITY;
   st->iters = 0;
   st->done = 0;
@@ -685,7 +700,8 @@ int iterate(gg_graph *g, Op op, int dir, const SliceLists *slices, PrState *st, 
           seg_rows_launch(op, offs, g->n, g->m, parts, carry, done, g->opt.expand_grid, s);
       }
       if (offset_out)
-        hipLaunchKernelGGL(k_adj_finalize, dim3(1), dim3(kWave), 0, s, st, tol, max_iter, g->n, (double)op.d);
+        hipLaunchKernelGGL(k_adj_finalize, dim3(1), dim3(kWave), 0, s, st, tol, max_iter, g->n, (double)op.d,
+                           shift_last(op.d));
       else
         hipLaunchKernelGGL(k_pr_finalize, dim3(1), dim3(kWave), 0, s, st, tol, max_iter);
     }
@@ -743,7 +759,7 @@ int gg_pagerank(gg_graph *g, float damping, const float *teleport, double tol_l1
   GG_HIP(fill_async<unsigned char>(reinterpret_cast<unsigned char *>(st), 0, sizeof(PrState), s));
   hipLaunchKernelGGL(k_pr_init, dim3(grid_for(n, kRowBlock, 4096)), dim3(kRowBlock), 0, s, r0,
                      weighted ? nullptr : x0, tele, g->pr[0].as<float>(), n, st, 0, (const float *)nullptr);
-  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(kWave), 0, s, st, 0);
+  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(kWave), 0, s, st, 0, 0);
   GG_HIP(hipGetLastError());
   PrForwardOp op{};
   op.off = g->dg.column_offsets;
@@ -834,7 +850,7 @@ int gg_pagerank_adjoint(gg_graph *g, float damping, const float *rank, const flo
   GG_HIP(fill_async<unsigned char>(reinterpret_cast<unsigned char *>(st), 0, sizeof(PrState), s));
   hipLaunchKernelGGL(k_pr_init, dim3(grid_for(n, kRowBlock, 4096)), dim3(kRowBlock), 0, s, l0, (float *)nullptr,
                      (const float *)nullptr, g->pr[0].as<float>(), n, st, 1, d_c);
-  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(kWave), 0, s, st, 1);
+  hipLaunchKernelGGL(k_pr_start, dim3(1), dim3(kWave), 0, s, st, 1, tol_l1 < kSettled);
   GG_HIP(hipGetLastError());
   PrAdjointOp op{};
   op.off = g->dg.row_offsets;

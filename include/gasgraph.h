@@ -216,7 +216,10 @@ int gg_pagerank(gg_graph *g, float damping, const float *teleport,
  * ranks: grad_w (m, CSR order) = dL/dw for the raw F32 values (or dL/dP_uv
  * when the graph has no F32 values); grad_t (n) = dL/dt.  Either output may
  * be NULL.  The adjoint iteration stops when its L1 residual is at most
- * tol_l1 * ||c||_1.  With GG_OUT_DEVICE every array argument (rank, c and
+ * tol_l1 * ||c||_1; stats->residual is that residual or an upper bound of it
+ * that meets the tolerance.  After max_iter sweeps: GG_ERR_NOT_CONVERGED, with
+ * the gradients of the plain iterate of that many sweeps written, and its L1
+ * residual.  With GG_OUT_DEVICE every array argument (rank, c and
  * the outputs) is a device pointer.  No reference counterpart. */
 int gg_pagerank_adjoint(gg_graph *g, float damping, const float *rank,
                         const float *c, double tol_l1, int32_t max_iter,

@@ -468,3 +468,76 @@ def test_adjoint_gradient_row_lengths(gpu_available, weighted):
         if k > 1:  # a single edge's weight does not matter: its gradient is 0 but for rounding
             assert np.linalg.norm(gw[row] - gw64[row]) / np.linalg.norm(gw64[row]) < 1e-4, k
     assert np.linalg.norm(gw - gw64) / np.linalg.norm(gw64) < 1e-4
+
+
+def adjoint_graph(kind):
+    if kind == "forest":
+        return gg.gen_erdos_renyi(100000, 60000, 3)
+    if kind == "sparse":
+        return gg.gen_erdos_renyi(2000, 6000, 3)
+    if kind == "lattice":
+        return gg.gen_lattice(40, seed=4)
+    if kind == "pairs":
+        return csr_from_edges(400, np.arange(400), np.arange(400) ^ 1)
+    return gg.gen_rmat(12, 16, undirected=False, seed=63)
+
+
+def plain_adjoint(c, cv, d, sweeps=None, tol=0.0):
+    """FP64 plain iteration from c, unweighted: its vector, the L1 change of its
+    last sweep and the number of sweeps (as many as asked for, or until the
+    change is at most tol ||c||_1)."""
+    rows, deg = np.repeat(np.arange(c.n), c.degrees()), c.degrees()
+    lam, k = cv.astype(np.float64), 0
+    while True:
+        s = np.bincount(rows, lam[c.col_indices], c.n) / np.maximum(deg, 1)
+        new = cv + d * np.where(deg == 0, lam.sum() / c.n, s)
+        resid, lam, k = np.abs(new - lam).sum(), new, k + 1
+        if k == sweeps or (sweeps is None and resid <= tol * np.abs(cv).sum()):
+            return lam, resid, k
+
+
+@pytest.mark.parametrize("kind,loss,d,tol", [
+    ("forest", "ones", 0.95, 2e-7), ("forest", "pos", 0.85, 1e-8), ("sparse", "onehot", 0.85, 1e-8),
+    ("sparse", "ones", 0.85, 1e-9), ("lattice", "ones", 0.85, 1e-8), ("lattice", "pos", 0.85, 0.0),
+    ("pairs", "pos", 0.85, 1e-9), ("sparse", "pos", 0.3, 0.0), ("rmat", "pos", 0.5, 1e-9)])
+def test_adjoint_ends_where_plain_sweeps_end(gpu_available, kind, loss, d, tol):
+    """Losses and tolerances at the level of FP32 rounding, which plain FP32
+    sweeps meet because their vectors settle: the run meets them as well, within
+    the sweeps allowed.  Error as in the other adjoint tests."""
+    c = adjoint_graph(kind)
+    rng = np.random.default_rng(7)
+    cv = {"ones": np.ones(c.n), "pos": rng.random(c.n), "onehot": np.eye(1, c.n, c.n // 2)[0]}[loss]
+    cv = cv.astype(np.float32)
+    with gg.Graph(c, directed=True) as g:
+        _, gt, st = g.pagerank_adjoint(np.full(c.n, 1.0 / c.n, np.float32), cv, damping=d, tol_l1=tol)
+    assert st["residual"] <= tol * np.abs(cv, dtype=np.float64).sum()
+    lam = plain_adjoint(c, cv, np.float32(d).astype(np.float64), tol=1e-14)[0]
+    bound = d / (1 - d) * tol * np.abs(cv).sum() + 2.0**-22 / (1 - d) * np.abs(lam).max()
+    assert np.abs(gt - (1 - np.float32(d)) * lam).max() <= (1 - d) * bound + 2.0**-23 * np.abs(gt).max()
+
+
+@pytest.mark.parametrize("kind", ["rmat", "sparse", "lattice", "pairs"])
+@pytest.mark.parametrize("sweeps", [1, 2, 5, 17])
+def test_adjoint_at_its_limit(gpu_available, kind, sweeps):
+    """max_iter sweeps end with GG_ERR_NOT_CONVERGED, and the outputs hold the
+    plain iterate of that many sweeps and its L1 residual, whatever the shift
+    had added: FP32 rounding of vectors of the fixed point's size, amplified by
+    1 / (1 - d)."""
+    import ctypes as C
+
+    from gpugraph_amd import _abi
+
+    d = 0.85
+    c = adjoint_graph(kind)
+    cv = np.random.default_rng(11).random(c.n).astype(np.float32) + np.float32(0.5)
+    rank = np.full(c.n, 1.0 / c.n, np.float32)
+    gt, st = np.full(c.n, np.nan, np.float32), _abi.Stats()
+    ptr = lambda a: C.c_void_p(a.ctypes.data)  # noqa: E731
+    with gg.Graph(c, directed=True) as g:
+        rc = g.lib.gg_pagerank_adjoint(g.h, d, ptr(rank), ptr(cv), 1e-9, sweeps, None, ptr(gt), 0, C.byref(st))
+    assert rc == _abi.GG_ERR_NOT_CONVERGED and st.iterations == sweeps
+    lam, resid, _ = plain_adjoint(c, cv, d, sweeps=sweeps)
+    size = plain_adjoint(c, cv, d, tol=1e-12)[0].max()
+    rounding = 2.0**-22 / (1 - d) * size
+    assert np.abs(gt - (1 - d) * lam).max() <= (1 - d) * rounding + 2.0**-23 * size
+    assert abs(st.residual - resid) <= 2 * c.n * rounding
