@@ -274,8 +274,10 @@ class Graph:
         return out, st.as_dict()
 
     def cc(self, hook: bool = False, gas: bool = False, flags: int = 0, out=None):
-        """CC labels (gg_cc): label propagation (default), through the generic
-        GAS path (gas=True) or by hooking (hook=True)."""
+        """CC labels (gg_cc): by default hooking on graphs of 2^17 vertices and
+        more and label propagation, ended by hooking, on smaller ones; label
+        propagation throughout under an iteration limit (iter_num < n); through
+        the generic GAS path (gas=True) or by hooking (hook=True)."""
         st = _abi.Stats()
         f = flags | (_abi.GG_CC_HOOK if hook else 0) | (_abi.GG_CC_GAS if gas else 0)
         out, ptr = self._out(out, np.int32, f)

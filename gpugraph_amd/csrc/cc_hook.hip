@@ -25,7 +25,7 @@
 // The link pass is bound by its chains of dependent loads and by atomics on
 // the roots that most trees join (a wave sends one hook per pair of roots, and
 // a root is read again before its CAS: 2.4 -> 0.09 ms on an R-MAT), the others
-// by latency and launches: each moves about 8 n bytes, against 8 m for hooking
+// by latency and launches: each moves 8-16 n bytes, against 8 m for hooking
 // every edge.  Per call, against label propagation / hooking every edge:
 // 2048 x 2048 lattice (4.2M vertices, 10M edges) 12.4 / 0.66 -> 0.42 ms; R-MAT
 // of 1.5M vertices and 35M edges 0.92 -> 0.16-0.20 ms; of 4.2M vertices and 128M
@@ -38,15 +38,18 @@
 // vertex of the same tree; a hook decides by the CAS, whose returned value is
 // current, and path halving only ever replaces the parent of a vertex that
 // is not a root by a smaller vertex of the same tree.  (System-scope loads,
-// which bypass the L2, made each walk step a trip past it.)  Halving
-// stores are agent-scope: two XCDs that halve the same path may store
-// different values, and with plain stores each XCD's L2 kept its own value
-// across the kernel's end, so that a later kernel could see a path shorter
-// than the one in memory.  Words with one writer per kernel take plain stores.
+// which bypass the L2, made each walk step a trip past it.)  Halving stores are
+// agent-scope: with plain ones, where workgroups of several XCDs halve the same
+// path and store different values to one word in a kernel, runs ended with
+// labels that were not roots, and with agent-scope ones none did; why was not
+// established.  Words with one writer per kernel, or writers that all store the
+// same value, take plain stores.
 // Symmetric (undirected) graphs only.
 //
-// Byte model: 28 n (init 12, link and flatten 16) + 8 n (labels) + 8 per edge
-// of the rest pass.
+// Byte model: 44 n (init 12: offsets, first neighbour, parent; two flattens of
+// 8: parent and its parent; link 16: offsets, second neighbour, two parents),
+// the rest 12 n (flatten, parent) and 8 per edge (neighbour, its parent), the
+// labels 8 n.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -304,6 +307,7 @@ int cc_hook_finish(gg_graph *g, int32_t *parent, bool linked) {
     hipLaunchKernelGGL(k_cc_labels, grid, block, 0, s, parent, n);
     GG_HIP(hipGetLastError());
   }
+  g->prof.add_bytes("cc.rest", 12.0 * n);  // the caller adds its edges, read back after
   g->prof.add_bytes("cc.labels", 8.0 * n);
   return GG_OK;
 }
@@ -340,14 +344,14 @@ int cc_hooking(gg_graph *g, int32_t *label_out, uint32_t flags, gg_stats *stats)
   const int64_t rest = g->h64()[32];
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, e0, e1);
-  g->prof.add_bytes("cc.link", 28.0 * n);
+  g->prof.add_bytes("cc.link", 44.0 * n);
   g->prof.add_bytes("cc.rest", 8.0 * (double)rest);
   finish_profile(g);
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     stats->iterations = 3;
     stats->edges_inspected = std::min<int64_t>(2 * (int64_t)n, g->m) + rest;
-    stats->alg_bytes = 36.0 * n + 8.0 * (double)rest;
+    stats->alg_bytes = 44.0 * n + cc_finish_bytes(n, rest);
     stats->gpu_ms = ms;
     stats->reached_vertices = n;  // every vertex has a component
     stats->reached_edges = g->m;

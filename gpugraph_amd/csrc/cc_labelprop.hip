@@ -398,7 +398,7 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
   if (hooked) {
     GG_TRY(read_counters(g, 33));
     rest = g->h64()[32];
-    g->prof.add_bytes("cc.rest", 8.0 * (double)rest + 8.0 * n);
+    g->prof.add_bytes("cc.rest", 8.0 * (double)rest);
   }
   const double F = (double)h.frontier_total;
   const double bytes = 12.0 * n + words * 8.0 + 16.0 * (double)h.push_frontier + 8.0 * (double)h.edges +
@@ -410,7 +410,7 @@ int cc_label_propagation(gg_graph *g, int32_t *label_out, uint32_t flags, gg_sta
     stats->iterations = h.iters + (hooked ? 1 : 0);
     stats->pull_iterations = h.pulls;
     stats->edges_inspected = (int64_t)h.edges + rest;
-    stats->alg_bytes = bytes + (hooked ? 16.0 * n + 8.0 * (double)rest : 0.0);
+    stats->alg_bytes = bytes + (hooked ? cc_finish_bytes(n, rest) : 0.0);
     stats->gpu_ms = ms;
     stats->reached_vertices = n;  // every vertex has a label
     stats->reached_edges = g->m;

@@ -109,11 +109,16 @@ int get_problem(gg_graph *g, Problem<P> **out) {
 // Algorithmic bytes of iterations with frontier F, edges E, next frontier N
 // (per iteration, or summed over a run: the model is linear).
 template <class P>
+constexpr double edge_bytes() {  // sssp: target, weight, distance; the others: neighbour and one word of it
+  return std::is_same<P, sssp>::value ? 12 : 8;
+}
+template <class P>
 double iteration_bytes(double F, double E, double N) {
-  if (std::is_same<P, sssp>::value) return 16 * F + 12 * E + 8 * N;
-  if (std::is_same<P, cc>::value || std::is_same<P, cc_weak>::value) return 16 * F + 8 * E + 8 * N;
-  if (std::is_same<P, bfs>::value || std::is_same<P, bfs_reverse>::value) return 12 * F + 8 * E + 8 * N;
-  return 12 * F + 12 * E + 8 * N;  // pagerank: gather reads ri + rank + outdeg per in-edge
+  const double e = edge_bytes<P>() * E;
+  if (std::is_same<P, sssp>::value) return 16 * F + e + 8 * N;
+  if (std::is_same<P, cc>::value || std::is_same<P, cc_weak>::value) return 16 * F + e + 8 * N;
+  if (std::is_same<P, bfs>::value || std::is_same<P, bfs_reverse>::value) return 12 * F + e + 8 * N;
+  return 20 * F + e + 8 * N;  // pagerank: the apply also reads the degree and writes rank / degree
 }
 
 template <class P>
@@ -160,7 +165,7 @@ int run_program(gg_graph *g, int num_srcs, int *srcs, typename P::DataType *out,
       const double b = iteration_bytes<P>(r);
       const std::string base = std::string(Slot<P>::name) + ".";
       // Edge traffic to the expand kernel, per-vertex traffic to the count pass.
-      const double fb = b - (std::is_same<P, cc>::value ? 8 : 12) * (double)r.edges - 8.0 * r.next;
+      const double fb = b - edge_bytes<P>() * (double)r.edges - 8.0 * r.next;
       g->prof.add_bytes((base + (r.lbs ? "lbs_expand" : "tiered_expand")).c_str(), b - fb);
       g->prof.add_bytes((base + (r.lbs ? "lbs_count" : "prologue")).c_str(), fb);
     }
@@ -244,15 +249,16 @@ int sssp_core(gg_graph *g, int32_t src, int32_t *dist, uint32_t flags, gg_stats 
   return run_program<sssp>(g, 1, &s, dist, flags, stats, sssp::INIT_VALUE, true);
 }
 
-// gg_cc's default from this many vertices on: sampled hooking.  Label
-// propagation takes an iteration per unit of diameter over every edge;
-// hooking is faster at every size measured (2^17-vertex R-MAT 0.32 -> 0.12 ms,
-// 400 x 400 lattice 3.4 -> 0.10 ms, 200 x 200 lattice 2.9 -> 0.08 ms).  Below,
-// label propagation still runs its first 16 iterations (10-20 us each), since
-// the iteration counts of small runs are read as the propagation's depth, and
-// hooking ends what is left (200 x 200 lattice 2.9 -> 0.47 ms); a limit
-// on the iterations (iter_num < n) keeps it throughout, its partial labels
-// being what such a call asks for.
+// gg_cc's default from this many vertices on: sampled hooking.  The line is not
+// one of speed: hooking is faster at every size measured (a call, labels left on
+// the device, default / hooking: 4096-vertex Erdos-Renyi 192 / 71 us,
+// 65k-vertex R-MAT 212 / 123, 200 x 200 lattice 330 / 81; 2^17-vertex R-MAT,
+// label propagation / hooking, 320 / 120).  Below it the default stays label
+// propagation for the statistics that calls on small graphs have had
+// (iterations and pull_iterations of the propagation, where it ends within its
+// first replay of 16); what is left after that hooking ends (200 x 200
+// lattice 2.9 ms without).  A limit on the iterations (iter_num < n) keeps label
+// propagation throughout, its partial labels being what such a call asks for.
 constexpr int32_t kCcHookMin = 1 << 17;
 
 int cc_core(gg_graph *g, int32_t *label, uint32_t flags, gg_stats *stats) {

@@ -398,6 +398,7 @@ int batch_bfs(gg_graph *g, const int32_t *sources, int32_t num, int32_t *depth_o
 // as cc_hooking's first half leaves it.
 int cc_hooking(gg_graph *g, int32_t *label, uint32_t flags, gg_stats *stats);
 int cc_hook_finish(gg_graph *g, int32_t *parent, bool linked);
+inline double cc_finish_bytes(int32_t n, int64_t rest) { return 20.0 * n + 8.0 * (double)rest; }
 // Symmetry / value-symmetry check of an undirected graph (sets mirror_ok,
 // values_asymmetric); GG_ERR_INVALID when the CSR is provably not symmetric.
 int check_undirected(gg_graph *g);

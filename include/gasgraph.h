@@ -62,7 +62,7 @@ extern "C" {
 #define GG_OUT_DEVICE 1u        /* output pointers are device memory */
 #define GG_INSTRUMENT 2u        /* record per-kernel HIP-event timings (gg_profile_*) */
 #define GG_BFS_PUSH_ONLY 4u     /* BFS through the generic GAS program path (no bottom-up) */
-#define GG_CC_HOOK 8u           /* CC by min-id hooking + pointer jumping instead of label propagation */
+#define GG_CC_HOOK 8u           /* CC by min-id hooking + pointer jumping at every size */
 #define GG_SSSP_GAS 16u         /* SSSP through the generic GAS program path (reference semantics) */
 #define GG_CC_GAS 32u           /* CC label propagation through the generic GAS program path */
 #define GG_BFS_REVERSE 64u      /* BFS over in-edges (hops to src), GAS path, EXPAND_IN_EDGES */
@@ -99,14 +99,14 @@ typedef struct gg_options {
 
 /* Per-run statistics (the reference prints these with INSTRUMENT/verbose). */
 typedef struct gg_stats {
-  int32_t iterations;       /* GAS iterations (BFS levels) */
+  int32_t iterations;       /* GAS iterations (BFS levels; CC by hooking: its passes) */
   int32_t pull_iterations;  /* of which bottom-up / pull steps */
   int64_t reached_vertices; /* vertices with a final value != sentinel */
   int64_t reached_edges;    /* sum of CSR out-degree over reached vertices (GTEPS numerator) */
   int64_t edges_inspected;  /* edges actually examined, summed over iterations */
   double alg_bytes;         /* algorithmic HBM bytes of the run (byte model of the kernel set) */
   double gpu_ms;            /* HIP-event time of the device section */
-  double residual;          /* PageRank: last L1 residual (FP64); else 0 */
+  double residual;          /* PageRank: last L1 residual (FP64), adjoint: or a bound of it; else 0 */
 } gg_stats;
 
 /* ---- library ------------------------------------------------------------ */
@@ -187,8 +187,8 @@ int gg_sssp(gg_graph *g, int32_t src, int32_t *dist, uint32_t flags,
  * EnactIterativeSearch with Program = cc (Algorithms/CC/cc.h:32-349; driver
  * cc.cu:291-292).  Default: below 2^17 vertices the program's label
  * propagation as a device-driven loop (hipGraph replays), ended by hooking
- * when 16 iterations have not been enough; from there on hooking, with
- * stats->iterations its passes; with iter_num < n label propagation
+ * when 16 iterations have not been enough (which counts as one more); from
+ * there on hooking, with stats->iterations its passes; with iter_num < n label propagation
  * throughout.  GG_CC_GAS: the program through the generic GAS path;
  * GG_CC_HOOK: hooking + pointer jumping at every size.  Undirected graphs.
  * Hooking joins the ends of every entry, also where rows are not sorted and

@@ -4,7 +4,8 @@ benchmark runs them with (graphs stored renumbered by degree):
   R-MAT scale 22 undirected (4.19M vertices, 128M CSR entries): BFS, SSSP and
     CC (label propagation, hooking, the generic GAS program) bit-exact
     against the oracle.
-  2048 x 2048 percolated lattice: the three CC engines bit-exact.
+  2048 x 2048 percolated lattice: the three CC engines bit-exact.  (At these
+    sizes the default is hooking; an iteration limit keeps label propagation.)
   R-MAT scale 20 directed, 128 SSSP + 64 personalised PageRank instances in
     one batched run: 8 SSSP rows bit-exact, 4 PPR rows against the FP64
     oracle (L1 tolerances stated below); 128 batched BFS instances, 8 rows
@@ -66,6 +67,8 @@ def test_config2_cc(gpu_available, rmat22):
             for mode in ({}, {"hook": True}, {"gas": True}):
                 lab, st = g.cc(**mode)
                 np.testing.assert_array_equal(lab, exp, err_msg=f"reorder={reorder} {mode}")
+            g.set_options(iter_num=c.n - 1)
+            np.testing.assert_array_equal(g.cc()[0], exp, err_msg=f"reorder={reorder} label propagation")
 
 
 def test_config3_lattice_cc(gpu_available):
@@ -75,6 +78,10 @@ def test_config3_lattice_cc(gpu_available):
         for mode in ({}, {"hook": True}, {"gas": True}):
             lab, st = g.cc(**mode)
             np.testing.assert_array_equal(lab, exp, err_msg=str(mode))
+        g.set_options(iter_num=lat.n - 1)
+        lab, st = g.cc()
+        np.testing.assert_array_equal(lab, exp, err_msg="label propagation")
+        assert st["iterations"] > 32
     assert len(np.unique(exp)) > 1000  # percolation leaves many components
 
 

@@ -97,9 +97,10 @@ def test_expand_strategies_agree(gpu_available, threshold):
 
 
 def test_lattice_cc(gpu_available):
-    """The three CC engines on the percolated lattice (many iterations of
-    label propagation: several graph replays of the device-driven loop) and on
-    R-MAT with its hubs (wave-cooperative rows); expand grid and wave split
+    """The CC engines on the percolated lattice (the default's label
+    propagation ended by hooking after its first replay; label propagation to
+    the end, several replays of the device-driven loop; the GAS program; hooking)
+    and on R-MAT with its hubs (wave-cooperative rows); expand grid and wave split
     varied."""
     c = workloads.config3_lattice(side=256)
     exp, _ = oracle.cc(c.row_offsets, c.col_indices)
@@ -109,10 +110,14 @@ def test_lattice_cc(gpu_available):
             np.testing.assert_array_equal(lab, exp, err_msg=str(mode))
             assert st["reached_vertices"] == c.n
         lab, st = g.cc()
-        assert st["iterations"] > 16  # more than one replay of the captured loop
+        assert st["iterations"] > 16  # the first replay's, and hooking's pass
         g.set_options(expand_grid=64, wave_degree=2)
         lab, _ = g.cc()
         np.testing.assert_array_equal(lab, exp)
+        g.set_options(iter_num=c.n - 1)  # a limit: label propagation throughout
+        lab, st = g.cc()
+        np.testing.assert_array_equal(lab, exp)
+        assert st["iterations"] > 32 and st["pull_iterations"] > 16  # more than one replay of the captured loop
     r = gg.gen_rmat(14, 16, undirected=True, seed=25)
     with gg.Graph(r) as g:
         exp_r = oracle.cc(r.row_offsets, r.col_indices)[0]
