@@ -335,7 +335,7 @@ static hipError_t upload(gg_graph *g, void *dst, const void *src, size_t bytes) 
     (void)hipGetLastError();  // memory the runtime does not know
   } else if (at.type != hipMemoryTypeUnregistered) {
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, 4);
+    hipError_t e = GASengine::device_alloc(&p, 4);
     if (e == hipSuccess) e = hipFree(p);
     if (e != hipSuccess) return e;
   }
